@@ -1,0 +1,158 @@
+"""GPU parity of the wide GEMM's 2 x 2-wave tiles where they can go wrong: the first and last
+rows and columns of every tile size, a K of one, odd and half super-tiles, K splits, the
+output formats and alignments that leave the accumulators another way, swizzled activation
+scales.  The four-wave and generic kernels, themselves checked against the oracle, are the
+reference: whole-K sums are the same chain of MFMAs (equal bits); others meet the GEMM bar."""
+import pytest
+import torch
+
+from test_gpu_gemm import _act, _check, _weights
+
+pytestmark = pytest.mark.gpu
+
+
+def _options(ops, **fields):
+    from vllm_mach_amd import _lib
+    return _lib.GemmOptions(**fields)
+
+
+def _plan(M, N, K, fmt, block=0):
+    from vllm_mach_amd import _lib
+    return _lib.plan_name("mxl_gemm_plan_name", M, N, K, fmt, block)
+
+
+def _mx(pkg, oracle_mod, dev, M, N, K, fmt):
+    ops = pkg.ops
+    _, ws, stored = _weights(oracle_mod, N, K, fmt, 0.02, 5 + N + K)
+    tiled, tiled_s = ops.pack_weight(torch.from_numpy(stored).to(dev), torch.from_numpy(ws).to(dev), fmt)
+    a, sa = torch.ops.mach_amd.quantize_mxfp8(_act(M, K, 9 + M).to(dev), 0)
+    return a, sa, tiled, tiled_s
+
+
+def _block(pkg, dev, M, N, K):
+    g = torch.Generator().manual_seed(31 + M + K)
+    w = torch.randn(N, K, generator=g) * 0.02
+    wb = w.reshape(N // 128, 128, K // 128, 128)
+    sb = (wb.abs().amax(dim=(1, 3)) / 448.0).float()
+    wq = (wb / sb[:, None, :, None]).reshape(N, K).to(torch.float8_e4m3fn)
+    tiled, _ = pkg.ops.pack_weight(wq.to(dev), None, 0)
+    q, s = torch.ops.mach_amd.quantize_block_fp8(torch.randn(M, K, generator=g).bfloat16().to(dev))
+    return q, s, tiled, sb.to(dev)
+
+
+# M, N, K, fmt, tile (rows / 16, columns / 64) the planner takes, K splits
+TILES = [
+    (17, 12296, 1152, 0, "4,1", False),    # the fewest rows; N % 64 = 8; nine slices (2.25 super-tiles)
+    (20, 2560, 9216, 0, "4,1", True),
+    (600, 4100, 128, 2, "4,1", False),     # one slice; N % 16 = 4
+    (63, 18440, 768, 3, "4,2", False),     # N % 128 = 8, one and a half super-tiles
+    (257, 4104, 896, 3, "4,2", False),     # one row in the last row of tiles
+    (160, 6000, 2048, 0, "8,1", False),
+    (200, 1152, 14336, 3, "8,1", True),
+    (200, 9000, 1024, 0, "8,2", False),
+    (129, 17408, 5120, 2, "8,2", True),    # whole-K tiles and split remainder in one launch
+    (900, 10000, 384, 0, "8,4", False),    # less than a super-tile
+    (1090, 8200, 640, 0, "8,4", False),    # quarters of 41 tiles past a full round: 2 rows, 8 columns of the last
+    (1500, 18432, 512, 0, "16,4", False),  # one super-tile; quarters
+    (700, 18400, 2560, 2, "16,4", False),  # N % 256 = 224
+    (2000, 9000, 1280, 3, "16,4", False),  # quarters of 32 tiles: 80 rows, 40 columns of the last
+]
+
+
+@pytest.mark.parametrize("M,N,K,fmt,tile,split", TILES)
+def test_mx_tiles(pkg, oracle_mod, dev, monkeypatch, M, N, K, fmt, tile, split):
+    ops = pkg.ops
+    plan = _plan(M, N, K, fmt)
+    assert plan.startswith(f"gemm_wide_kernel<{fmt},{tile},false,false,2>")
+    assert plan.endswith("wide_tile_reduce_kernel") == split
+    a, sa, w, sw = _mx(pkg, oracle_mod, dev, M, N, K, fmt)
+    monkeypatch.setattr(ops, "_tuning", None)
+    y = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, None)
+    four = M >= 64 and K % 256 == 0
+    monkeypatch.setattr(ops, "_tuning", _options(ops, tile_n=2, splits=1, waves=4) if four else _options(ops, kernel=2))
+    ref = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, None)
+    if four and not split:
+        assert torch.equal(y, ref)
+    _check(y.float().cpu().numpy(), ref.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("M,N,K,tile,split", [
+    (17, 18432, 1024, "4,2", False),
+    (40, 2560, 9344, "4,1", True),      # 73 slices: the last stage is past K
+    (130, 18432, 640, "4,2", False),
+    (300, 18432, 2560, "8,2", False),
+    (1090, 7552, 1280, "8,2", False),   # quarters of 19 tiles, 2 rows of the last
+])
+def test_block_fp8_tiles(pkg, dev, monkeypatch, M, N, K, tile, split):
+    ops = pkg.ops
+    plan = _plan(M, N, K, 0, 1)
+    assert plan.startswith(f"gemm_wide_kernel<0,{tile},true,false,2>")
+    assert plan.endswith("wide_tile_reduce_kernel") == split
+    q, s, w, sb = _block(pkg, dev, M, N, K)
+    monkeypatch.setattr(ops, "_tuning", None)
+    y = torch.ops.mach_amd.block_fp8_gemm(q, s, w, sb, N, K, None)
+    four = M >= 64 and K % 256 == 0
+    monkeypatch.setattr(ops, "_tuning", _options(ops, tile_n=2, splits=1, waves=4) if four else _options(ops, kernel=2))
+    ref = torch.ops.mach_amd.block_fp8_gemm(q, s, w, sb, N, K, None)
+    if four and not split:
+        assert torch.equal(y, ref)
+    _check(y.float().cpu().numpy(), ref.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("N", [640, 642, 641])       # columns of 16-, 4- and 2-byte alignment
+@pytest.mark.parametrize("out_dtype,alpha,bias,pad", [(0, 1.0, False, 0), (0, 1.0, True, 8), (1, 0.5, False, 3),
+                                                      (0, 1.0, False, 1)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_tile_outputs(pkg, oracle_mod, dev, N, out_dtype, alpha, bias, pad, splits):
+    """The output forms of a 128 x 128 tile and of its split reduce: element format, scale,
+    bias, row stride and odd widths, against the four-wave kernel (equal bits)."""
+    from vllm_mach_amd import _lib
+    M, K, fmt = 200, 2304, 0
+    a, sa, w, sw = _mx(pkg, oracle_mod, dev, M, N, K, fmt)
+    b = (torch.randn(N, generator=torch.Generator().manual_seed(2)) * 0.5).bfloat16().to(dev) if bias else None
+    got = []
+    for waves in (4, 8):
+        o = _options(pkg.ops, tile_n=2, splits=splits, waves=waves, out_dtype=out_dtype, alpha=alpha)
+        nbytes = _lib.query("mxl_gemm_workspace_bytes_ex", M, N, K, fmt, 0, _lib.options_ptr(o))
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+        out = torch.full((M, N + pad), 7.0, dtype=torch.float16 if out_dtype else torch.bfloat16, device=dev)
+        _lib.call("mxl_mx_gemm_ex", a.data_ptr(), sa.data_ptr(), M, w.data_ptr(), sw.data_ptr(), N, K, fmt,
+                  None if b is None else b.data_ptr(), out.data_ptr(), N + pad, ws.data_ptr(), nbytes,
+                  _lib.options_ptr(o), torch.cuda.current_stream(dev).cuda_stream)
+        got.append(out)
+    assert torch.equal(got[0], got[1])
+    assert bool((got[1][:, N:] == 7.0).all())  # nothing past the row
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 2560), (200, 1024, 2304), (70, 512, 256)])
+def test_tiles_read_swizzled_scales(pkg, oracle_mod, dev, M, N, K):
+    from vllm_mach_amd import _lib
+    a, sa, w, sw = _mx(pkg, oracle_mod, dev, M, N, K, 2)
+    swz = torch.empty(_lib.query("mxl_swizzled_scale_bytes", M, K), dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    _lib.call("mxl_swizzle_scales", sa.data_ptr(), M, K, swz.data_ptr(), stream)
+    got = []
+    for layout, scales in ((0, sa), (1, swz)):
+        o = _options(pkg.ops, sa_layout=layout, tile_n=2, splits=1, waves=8)
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+        _lib.call("mxl_mx_gemm_ex", a.data_ptr(), scales.data_ptr(), M, w.data_ptr(), sw.data_ptr(), N, K, 2, None,
+                  out.data_ptr(), N, None, 0, _lib.options_ptr(o), stream)
+        got.append(out)
+    assert torch.equal(got[0], got[1])
+
+
+def test_noalloc_takes_a_plan_past_its_scratch(pkg, oracle_mod, dev):
+    """A shape whose plan splits K past the no-allocation scratch, though the four-wave plan
+    fits it (so the entry point takes the shape): runs whole-K."""
+    from vllm_mach_amd import _lib
+    M, N, K, fmt = 200, 9216, 32768, 0
+    assert _lib.query("mxl_gemm_workspace_bytes_ex", M, N, K, fmt, 0, None) > _lib.query("mxl_noalloc_scratch_bytes")
+    codes = torch.randint(0, 0x70, (N, K), dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+    scales = torch.randint(118, 122, (N, K // 32), dtype=torch.uint8, device=dev)
+    w, sw = pkg.ops.pack_weight(codes, scales, fmt)
+    a, sa = torch.ops.mach_amd.quantize_mxfp8(_act(M, K, 3).to(dev), 0)
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    _lib.call("mxl_mx_gemm_noalloc", a.data_ptr(), sa.data_ptr(), M, w.data_ptr(), sw.data_ptr(), N, K, fmt, None,
+              out.data_ptr(), N, torch.cuda.current_stream(dev).cuda_stream)
+    ref = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, None)
+    _check(out.float().cpu().numpy(), ref.float().cpu().numpy())

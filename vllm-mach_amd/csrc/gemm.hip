@@ -553,32 +553,45 @@ GemmOptions with_override(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
 }
 }  // namespace
 
-static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o,
-                          DensePlan& d);
+static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o, DensePlan& d,
+                          bool four_wave = false);
 
 static bool plan_dense(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o, DensePlan& d) {
   return plan_dense_as(M, N, K, fmt, block, with_override(M, N, K, fmt, block, o), d);
 }
 
-static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o,
-                          DensePlan& d) {
+// (four_wave: the plan of the four-wave tiles alone, whatever the 2 x 2-wave ones would do)
+static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o, DensePlan& d,
+                          bool four_wave) {
   const bool stream_ok = stream_gemm_eligible(M, K, block);
   const bool wide_ok = wide_gemm_eligible(M, K) && (!block || K <= int64_t(128) * kWideBlockStages);
   const bool chunk_ok = !block && chunk_gemm_eligible(M, K, fmt);
+  const bool tiles_ok = !four_wave && M > 16 && wide_tiles_eligible(M, N, K, block);
   // Short K over few n-tiles: the generic kernel splits K over the waves of one workgroup
   // and writes bf16 directly, where the wide kernel needs a K split and its reduce to fill
   // the CUs.  Measured by a per-shape sweep over every kernel, tile and split (µs, generic
   // against the wide or K-chunked pick): MXFP8 2048 x 2048 at M = 64 / 128 / 256 6.5 /
   // 7.5 / 8.5 against 8.6 / 8.7 / 13.0, W6A8 N = 512 and 2048, K = 2048 at M = 64..128
   // 5.9-7.2 against 8.1-8.4.
-  const bool generic_pref = !block && M > 32 && M <= 256 && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128;
+  // At 17 to 63 rows it keeps the small weights of a short K (us, generic against 2 x 2-wave tiles:
+  // 24 rows W6A8 of 6144 x 2048 6.8 against 7.7, 20 rows block-FP8 of 512 x 3968 6.0 against 7.6;
+  // past it 32 rows of 4864 x 2304 10.3 against 8.4, 38 of 17856 x 512 8.5 against 6.2, 34 of 256 x
+  // 5760 9.6 against 8.5); at 129 to 256 rows the tiles win (256 of 2048 x 2048 8.6 against 7.5).
+  // The chunked kernel beat the four-wave tiles; the 2 x 2-wave ones pass it wherever it was chosen
+  // (W6A8 4608 x 2048 at 72 / 96 / 128 rows 7.9 / 8.0 / 8.4 against 11.9 / 11.9 / 12.1).  It keeps
+  // the plans of all eight m-tiles, which callers hold by name; a registered entry picks the tiles there.
+  const bool chunk_pref = chunk_ok && chunk_gemm_preferred(M, N, K) && (M > 112 || !tiles_ok);
+  const bool generic_pref =
+      (!block && M > 32 && M <= (four_wave ? 256 : 128) && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128) ||
+      (M < 64 && K >= 1024 && N * K <= (K <= 2048 ? int64_t(12) << 20 : K <= 4096 ? int64_t(4) << 20 : 0));
   d.kernel = o.kernel == kAuto
                  ? (stream_ok                                        ? kStream
-                    : chunk_ok && chunk_gemm_preferred(M, N, K)      ? kChunk
-                    : generic_pref || !wide_ok                       ? kGeneric
+                    : chunk_pref                                     ? kChunk
+                    : generic_pref || !(wide_ok || tiles_ok)         ? kGeneric
                                                                      : kWide)
                  : o.kernel;
-  if ((d.kernel == kStream && !stream_ok) || (d.kernel == kWide && !wide_ok) || (d.kernel == kChunk && !chunk_ok) ||
+  if ((d.kernel == kStream && !stream_ok) || (d.kernel == kWide && !wide_ok && (o.kernel == kWide || !tiles_ok)) ||
+      (d.kernel == kChunk && !chunk_ok) ||
       (d.kernel != kStream && d.kernel != kWide && d.kernel != kGeneric && d.kernel != kChunk))
     return false;
   if (d.kernel == kChunk) {
@@ -587,32 +600,13 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
     return true;
   }
   if (d.kernel == kWide) {
-    if (block && o.tile_n == 0 && o.waves == 0 && o.splits == 0 && !o.hybrid && o.tile_m == 0) {
-      // Block-FP8: eight waves (two per SIMD, so one wave's per-K128 folds run under the
-      // other's MFMAs) on 128 x 128 tiles, which fit their registers.  Measured at c3 (N =
-      // 18432, K = 2560; µs, four-wave pick -> this): M = 128 23.4 -> 20.3, M = 256 37.2 ->
-      // 33.7 (one full round plus split remainder), M = 512 58.6 -> 55.5 (three rounds: the
-      // split remainder after two full rounds measured 63.7).
-      // At most 64 rows: 64-row tiles on four waves (c3 M = 64: 16.2 against 19.7 µs for
-      // half-empty 128-row tiles on eight).
-      GemmOptions o2 = o;
-      o2.tile_n = 2;
-      if (M <= 64) o2.tile_m = 4;
-      d.wide = wide_config(M, N, K, fmt, o2);
-      if (d.wide.dp_tiles >= 2 * (int64_t)cu_count()) {
-        const int mt = d.wide.MT;
-        d.wide = WideConfig{2, 1, (K + kTileK - 1) / kTileK};
-        d.wide.MT = mt;
-      }
-      d.wide.WM = d.wide.MT == 8 ? 2 : 1;
+    const bool auto_tile = o.tile_n == 0 && o.splits == 0 && o.waves == 0 && o.tile_m == 0 && !o.hybrid;
+    if (auto_tile && tiles_ok) {
+      d.wide = wide_tiles_config(M, N, K, fmt, block);
     } else {
       d.wide = wide_config(M, N, K, fmt, o);
-      if (block && d.wide.NT == 4) d.wide.WM = 1;  // no eight-wave block-FP8 tile of four n-tiles per wave
-      // MX 128 x 128 tiles: eight waves, bit-identical, measured 1-3 % faster where the
-      // model picks them (c2 M = 512 29.2 -> 28.5 µs, c4 M = 128 35.1 -> 34.0, M = 256
-      // 46.5 -> 46.2); 64-column tiles measured slower with eight waves
-      const bool auto_tile = o.tile_n == 0 && o.splits == 0 && o.waves == 0 && o.tile_m == 0 && !o.hybrid;
-      if (!block && auto_tile && d.wide.NT == 2 && d.wide.MT == 8) d.wide.WM = 2;
+      // no 2 x 2-wave block-FP8 tile of 256 columns
+      if (d.wide.WM == 2 && ((block && d.wide.NT == 4) || !wide_tiles_eligible(M, N, K, block))) d.wide.WM = 1;
     }
     d.need = wide_workspace_bytes(d.wide, M, N);
   } else if (d.kernel == kGeneric) {
@@ -665,9 +659,9 @@ static int gemm_common(const void* a, const void* sa, int64_t M, const void* w_t
   } else if (d.kernel == kWide) {
     WideConfig wc = d.wide;
     if (!room) {
-      const int mt = wc.MT;
       wc = WideConfig{wc.NT, 1, (K + kTileK - 1) / kTileK};  // no room: skip the K split
-      wc.MT = mt;
+      wc.MT = d.wide.MT;
+      wc.WM = d.wide.WM;
     }
     p.S = wc.S;
     e = launch_gemm_wide(fmt, block, wc, p, 0, s);
@@ -815,9 +809,10 @@ extern "C" int mxl_mx_gemm_noalloc(const void* a, const void* sa, int64_t M, con
   MXL_CHECK_ARG(M >= 0 && N > 0 && K > 0 && K % 128 == 0, "%s: need N > 0, K %% 128 == 0 (M=%lld N=%lld K=%lld)", who,
                 (long long)M, (long long)N, (long long)K);
   if (M == 0) return MXL_OK;
-  // the plan mxl_mx_gemm makes for this shape; its split-K partials must fit the scratch
+  // The split-K partials of the four-wave plan must fit the scratch (the shapes this entry
+  // point takes); where the plan mxl_mx_gemm makes needs more, it runs without its K split.
   DensePlan d;
-  if (!plan_dense(M, N, K, w_fmt, false, GemmOptions(), d)) {
+  if (!plan_dense_as(M, N, K, w_fmt, false, with_override(M, N, K, w_fmt, false, GemmOptions()), d, true)) {
     set_error("%s: no kernel runs this shape (M=%lld, K=%lld)", who, (long long)M, (long long)K);
     return MXL_EUNSUPPORTED;
   }

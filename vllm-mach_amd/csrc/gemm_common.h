@@ -145,7 +145,7 @@ struct GemmOptions {
   int tile_n = 0;     // wide: NT in {1, 2, 4}; 0 auto
   int tile_m = 0;     // wide: MT in {4, 8}; 0 auto
   int hybrid = 0;     // wide, splits == 1: full rounds whole-K, the remainder split
-  int waves = 0;      // wide MX dense, 128-row tiles: 4 or 8 waves per workgroup; 0 auto
+  int waves = 0;      // wide dense, 128-row tiles: 4 (side by side) or 8 (2 x 2-wave tiles, two per CU); 0 auto
   int out_dtype = kOutBf16;  // output element format
   float alpha = 1.0f;        // output scale
 };
@@ -264,11 +264,14 @@ struct WideConfig {
   int64_t dp_tiles = 0;
   int S2 = 1;
   int64_t kt2 = 0;
-  int MT = 8;  // 16-row m-tiles per workgroup tile: 8 (128 rows) or 4 (64 rows)
-  int WM = 1;  // m-groups of four waves: 1, or 2 (eight waves, each half the tile's rows)
+  int MT = 8;  // 16-row m-tiles per workgroup tile: 8 (128 rows), 4, or 16 (two by two waves only)
+  int WM = 1;  // the four waves side by side (1) or two by two (2)
 };
 // The cost model's choice, or the options' tile / split overrides where given.
 WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptions& o = GemmOptions());
+// The 2 x 2-wave tiles (gemm_tile.hip): the shapes they take, and the time model's choice.
+bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block);
+WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool block);
 // Workspace bytes a configuration needs (split partials), 0 when none.
 int64_t wide_workspace_bytes(const WideConfig& c, int64_t M, int64_t N);
 bool wide_gemm_eligible(int64_t M, int64_t K);
@@ -284,8 +287,6 @@ constexpr int kGroupedStreamWideMT = 6;
 int cu_count();
 hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const GemmParams& p, int64_t num_experts,
                             hipStream_t s);
-
-
 
 // K-chunked weight-streaming kernel for up to 128 rows (gemm_chunk.hip), MX weights:
 // chunks of kChunkSuperTiles super-tiles, fp32 partials [chunks][M][N] when K has more

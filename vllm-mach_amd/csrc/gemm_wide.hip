@@ -1,5 +1,6 @@
 // Wide-tile, LDS-pipelined GEMM for prefill-sized M on gfx950 (MX, block-FP8,
-// dense and MoE-grouped).
+// dense and MoE-grouped): the four-wave tiles, the planner of the dense 2 x 2-wave tiles
+// (gemm_tile.hip; what the automatic dense plans run) and the split reduce of both.
 //
 // Workgroup tile: 128 rows x 64*NT columns (NT = 1, 2 or 4), four wavefronts.
 // Every wave owns all 8 m-tiles of the 128 rows and its own NT n-tiles; per
@@ -44,7 +45,7 @@
 // of the split leftovers, so no CU waits for a second launch.  The grouped variant
 // walks experts' row ranges (expert_offsets) on device, so the launch needs no
 // host-side counts.
-#include "gemm_common.h"
+#include "gemm_wide.h"
 
 // the copies set M0 (the LDS base of a global->LDS load) themselves
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -53,10 +54,9 @@ namespace mxl {
 
 namespace {
 
-template <int MT, int NT, bool BLOCK, int WM = 1>
+template <int MT, int NT, bool BLOCK>
 struct WideSlot {
   static_assert(MT == 4 || MT == 8, "64- or 128-row workgroup tiles");
-  static_assert(WM == 1 || (WM == 2 && MT == 8), "two m-groups of waves: 128-row tiles only");
   // MX with NT <= 2: the activation scales live in a separate ring of three
   // super-tile entries (16 MT rows x 16 bytes), filled a super-tile ahead, so a
   // copy moves 16 bytes per row instead of one dword from each row.
@@ -69,16 +69,12 @@ struct WideSlot {
   static constexpr int SLOTS = NT == 4 ? 3 : 4;             // 4 x 53 KiB would not fit the LDS
   static constexpr int SW = MT / 4;                         // scale waves: 0 .. SW - 1, 64 rows each
   static constexpr int RING_ENTRY = 256 * MT;               // scale ring entry: 16 MT rows x 16 bytes
-  // WM m-groups of four waves: wave w owns m-tiles (w / 4) MT / WM .. + MT / WM - 1 and the
-  // n-tiles of n-group w % 4.  Copies per wave per stage: its share of the A chunks, of its
-  // n-group's B chunks (one of the two per n-tile when WM = 2) and of their E8M0 scales (with
-  // one n-tile both waves of the group copy it: the same bytes to the same place); the scale
-  // waves also copy the activation scales.
-  static constexpr int WAVES = 4 * WM;
+  // Copies per wave per stage: its share of the A chunks, its n-tiles' two B chunks each and
+  // their E8M0 scales; the scale waves also copy the activation scales.
+  static constexpr int WAVES = 4;
   static constexpr int ACH = 2 * MT / WAVES;
-  static constexpr int BCH = 2 / WM;
-  static constexpr int SBC = BLOCK ? 0 : (WM == 1 ? NT : (NT >= 2 ? NT / 2 : 1));
-  static constexpr int COPIES = ACH + BCH * NT + SBC;
+  static constexpr int SBC = BLOCK ? 0 : NT;
+  static constexpr int COPIES = ACH + 2 * NT + SBC;
 };
 
 // Ring slots of the grouped variant, which runs two workgroups per CU.
@@ -117,11 +113,11 @@ __device__ __forceinline__ void wait_vm() {
 // outstanding load): LDS data is handed over by the explicit waits.
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-template <int MT, int NT, int WM = 1>
+template <int MT, int NT>
 struct WideLanes {
   // A chunk c = ACH wv + u (m-tile c / 2, rows 8 (c % 2) .. + 7): copy lane l reads row
   // 8 (c % 2) + l / 8, piece (l % 8) ^ a_swz(row), as row * lda + 16 piece
-  uint32_t a_off[2 * MT / (4 * WM)];
+  uint32_t a_off[MT / 2];
   uint32_t sa_off;    // MX: row * K/32; block-FP8: 4 row  (row = t % 16 MT)
   uint32_t sa_piece[4];  // scale ring: lane l of scale wave w reads dword l % 4 of row 4 MT j + 16 w + l / 4
   uint32_t sa_last[4];   // the same for the last super-tile when it is half (K % 512 = 256), from p.sa and
@@ -134,12 +130,11 @@ struct WideLanes {
 // the scale ring, waves 0 and 1 also copy piece j (32 rows) of the next
 // super-tile's activation scales (clamped inside K: a piece past the last
 // super-tile is never read).
-template <int FMT, int MT, int NT, bool BLOCK, int WM>
+template <int FMT, int MT, int NT, bool BLOCK>
 __device__ __forceinline__ void wide_copy(const GemmParams& p, uint8_t* slot, int64_t t, int wv, int lane,
-                                          const WideLanes<MT, NT, WM>& L, uint8_t* sa_ring) {
-  using S = WideSlot<MT, NT, BLOCK, WM>;
+                                          const WideLanes<MT, NT>& L, uint8_t* sa_ring) {
+  using S = WideSlot<MT, NT, BLOCK>;
   constexpr int CH = FmtTraits<FMT>::CH;
-  const int wn = WM == 1 ? wv : wv & 3, wm = WM == 1 ? 0 : wv >> 2;
   const int64_t kt = t >> 2;
   const int j = (int)(t & 3);
 #pragma unroll
@@ -154,10 +149,8 @@ __device__ __forceinline__ void wide_copy(const GemmParams& p, uint8_t* slot, in
   for (int n = 0; n < NT; ++n) {
     const uint8_t* tile = L.w_tile[n] + kt * (CH * 1024) + c0 * 1024;
 #pragma unroll
-    for (int h = 0; h < S::BCH; ++h) {
-      const int c2 = WM == 1 ? h : wm;
-      copy16(tile + c2 * 1024, (uint32_t)(lane * 16), lds_addr(slot + S::B + ((wn * NT + n) * 2 + c2) * 1024));
-    }
+    for (int h = 0; h < 2; ++h)
+      copy16(tile + h * 1024, (uint32_t)(lane * 16), lds_addr(slot + S::B + ((wv * NT + n) * 2 + h) * 1024));
   }
   if (S::SA_RING) {
     if (wv < S::SW) {
@@ -175,8 +168,7 @@ __device__ __forceinline__ void wide_copy(const GemmParams& p, uint8_t* slot, in
   if (!BLOCK) {
 #pragma unroll
     for (int n = 0; n < NT; ++n)
-      if (WM == 1 || NT == 1 || (n & 1) == wm)
-        copy4(L.sw_tile[n] + kt * 256, (uint32_t)(lane * 4), lds_addr(slot + S::SB + (wn * NT + n) * 256));
+      copy4(L.sw_tile[n] + kt * 256, (uint32_t)(lane * 4), lds_addr(slot + S::SB + (wv * NT + n) * 256));
   }
 }
 
@@ -193,18 +185,16 @@ struct WideRegs {
 
 // Read stage operands (slice j of its super-tile) from a slot: B fragments
 // and scales first, then the MT A fragments in MFMA order.
-template <int FMT, int MT, int NT, bool BLOCK, int WM>
+template <int FMT, int MT, int NT, bool BLOCK>
 __device__ __forceinline__ void wide_read(const uint8_t* slot, const uint8_t* sa_entry, int j, int wv, int lane,
-                                          int q, int r, WideRegs<MT / WM, NT, BLOCK>& x) {
-  using S = WideSlot<MT, NT, BLOCK, WM>;
-  constexpr int MTW = MT / WM;
-  const int wn = WM == 1 ? wv : wv & 3, i0 = WM == 1 ? 0 : (wv >> 2) * MTW;
+                                          int q, int r, WideRegs<MT, NT, BLOCK>& x) {
+  using S = WideSlot<MT, NT, BLOCK>;
   // FP6: the slice's 24 bytes start at byte 0 (even j) or 8 (odd j) of the first chunk
   const int odd = j & 1;
   const int o0 = 8 * odd, o1 = odd ? 1024 : 8, o2 = odd ? 1032 : 1024;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
-    const uint8_t* base = slot + S::B + (wn * NT + n) * 2048 + lane * 16;
+    const uint8_t* base = slot + S::B + (wv * NT + n) * 2048 + lane * 16;
     if (FMT == kE4M3) {
       const uint4 lo = *reinterpret_cast<const uint4*>(base);
       const uint4 hi = *reinterpret_cast<const uint4*>(base + 1024);
@@ -215,19 +205,18 @@ __device__ __forceinline__ void wide_read(const uint8_t* slot, const uint8_t* sa
       const uint2 d2 = *reinterpret_cast<const uint2*>(base + o2);
       x.b[n] = v8i{(int)d0.x, (int)d0.y, (int)d1.x, (int)d1.y, (int)d2.x, (int)d2.y, 0, 0};
     }
-    if (!BLOCK) x.sb[n] = slot[S::SB + (wn * NT + n) * 256 + lane * 4 + j];  // byte j: slice j
+    if (!BLOCK) x.sb[n] = slot[S::SB + (wv * NT + n) * 256 + lane * 4 + j];  // byte j: slice j
   }
 #pragma unroll
-  for (int i = 0; i < MTW; ++i) {
-    const int gi = i0 + i;  // the wave's i-th m-tile within the workgroup tile
-    const uint8_t* row = slot + S::A + gi * 2048 + (r >> 3) * 1024 + (r & 7) * 128;
+  for (int i = 0; i < MT; ++i) {
+    const uint8_t* row = slot + S::A + i * 2048 + (r >> 3) * 1024 + (r & 7) * 128;
     const int sw = a_swz(r);
     const uint4 lo = *reinterpret_cast<const uint4*>(row + 16 * (q ^ sw));        // K 16 q ..
     const uint4 hi = *reinterpret_cast<const uint4*>(row + 16 * ((q + 4) ^ sw));  // K 64 + 16 q ..
     x.a[i] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    if (S::SA_RING) x.sa[i] = sa_entry[(16 * gi + r) * 16 + 4 * j + q];
-    else if (!BLOCK) x.sa[i] = slot[S::SA + (16 * gi + r) * 4 + q];
-    else x.s4[i] = *reinterpret_cast<const float4*>(slot + S::SA + (16 * gi + 4 * q) * 4);
+    if (S::SA_RING) x.sa[i] = sa_entry[(16 * i + r) * 16 + 4 * j + q];
+    else if (!BLOCK) x.sa[i] = slot[S::SA + (16 * i + r) * 4 + q];
+    else x.s4[i] = *reinterpret_cast<const float4*>(slot + S::SA + (16 * i + 4 * q) * 4);
   }
 }
 
@@ -309,39 +298,25 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 
 }  // namespace
 
-struct WideGrid {
-  int64_t mblocks;       // dense: ceil(M / 16 MT); grouped: bound on sum_e ceil(rows_e / 16 MT)
-  int64_t nblocks;       // ceil(N / (64 NT))
-  int64_t kt_per_split;  // 512-wide super-tiles per split
-  int64_t num_experts;   // grouped only
-  int64_t tile0, tiles;  // dense: this launch covers output tiles [tile0, tile0 + tiles) (tile = nb * mblocks + mb)
-  // dense, one-launch hybrid: after its whole-K tile (tiles [0, tiles), bf16 out) workgroup
-  // L also runs unit L < rem_tiles * S2 of the remainder: tile rem_tile0 + L % rem_tiles,
-  // K split L / rem_tiles of kt2 super-tiles, into compact partials
-  int64_t rem_tile0, rem_tiles, kt2;
-  int S2;
-};
-
 // One output tile: rows [row_base, hi) of m-block rows (hi bounds the valid rows
 // of a grouped expert), n-block nb, K split `split`; w / sw are the expert's
 // weights.  The ring and the scale ring are the workgroup's LDS.
-template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED, int WM>
+template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED>
 __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int64_t row_base, int64_t hi,
                                           const uint8_t* w, const uint8_t* sw, int64_t nb, int64_t split,
                                           float* pdst, uint8_t* ring, uint8_t* sa_ring, float* sb_stage,
                                           int t, int lane, int wv, int r, int q) {
-  using S = WideSlot<MT, NT, BLOCK, WM>;
+  using S = WideSlot<MT, NT, BLOCK>;
   constexpr int C = S::COPIES;
-  constexpr int BM = 16 * MT, MTW = MT / WM;
-  const int wn = WM == 1 ? wv : wv & 3, wm = WM == 1 ? 0 : wv >> 2;
+  constexpr int BM = 16 * MT;
   auto a_row = [&](int64_t row) -> int64_t {
     if (row >= hi) row = hi - 1;  // padding rows copy a valid row; their outputs are not stored
     return (GROUPED && p.row_index) ? (int64_t)(p.row_index[row] / p.row_div) : row;
   };
   const int64_t ntiles_total = (p.N + 15) / 16;
-  const int64_t nt_wave = (nb * 4 + wn) * NT;
+  const int64_t nt_wave = (nb * 4 + wv) * NT;
   constexpr int CH = FmtTraits<FMT>::CH;
-  WideLanes<MT, NT, WM> L;
+  WideLanes<MT, NT> L;
 #pragma unroll
   for (int u = 0; u < S::ACH; ++u) {
     const int c = S::ACH * wv + u;               // the A chunk: m-tile c / 2, rows 8 (c % 2) .. + 7
@@ -385,9 +360,9 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
     }
   }
 
-  v4f acc[MTW][NT];
+  v4f acc[MT][NT];
 #pragma unroll
-  for (int i = 0; i < MTW; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[i][n] = v4f{0.f, 0.f, 0.f, 0.f};
 
@@ -410,8 +385,8 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
     // reads, copies or its prologue and epilogue.
     constexpr int R = kWideGroupedSlots;
     static_assert(4 % R == 0, "the four steps below rotate the slots");
-    if (tb < te) wide_copy<FMT, MT, NT, BLOCK, WM>(p, ring, tb, wv, lane, L, sa_ring);
-    WideRegs<MTW, NT, BLOCK> x;
+    if (tb < te) wide_copy<FMT, MT, NT, BLOCK>(p, ring, tb, wv, lane, L, sa_ring);
+    WideRegs<MT, NT, BLOCK> x;
 #define MXL_WIDE_STEP2(I_)                                                                              \
   {                                                                                                   \
     const int64_t tt = t0 + I_;                                                                       \
@@ -420,11 +395,11 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                            \
       wide_barrier();                                                                                 \
       if (tt + 1 < te)                                                                                \
-        wide_copy<FMT, MT, NT, BLOCK, WM>(p, ring + ((I_ + 1) % R) * S::BYTES, tt + 1, wv, lane, L, sa_ring); \
-      wide_read<FMT, MT, NT, BLOCK, WM>(ring + (I_ % R) * S::BYTES, sa_ring + ((tt >> 2) % 3) * S::RING_ENTRY, \
+        wide_copy<FMT, MT, NT, BLOCK>(p, ring + ((I_ + 1) % R) * S::BYTES, tt + 1, wv, lane, L, sa_ring); \
+      wide_read<FMT, MT, NT, BLOCK>(ring + (I_ % R) * S::BYTES, sa_ring + ((tt >> 2) % 3) * S::RING_ENTRY, \
                                         (int)(tt & 3), wv, lane, q, r, x);                           \
       if (BLOCK) x.sbv = sb_stage[tt - tb];                                                           \
-      wide_mfma<FMT, MTW, NT, BLOCK>(x, acc);                                                         \
+      wide_mfma<FMT, MT, NT, BLOCK>(x, acc);                                                         \
     }                                                                                                 \
   }
     // four steps per iteration: tb is a multiple of 4, so each step's slice index
@@ -441,11 +416,11 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
     // prologue: stages tb .. tb + R - 1 fill the ring; stage tb is read into registers
 #pragma unroll
     for (int k = 0; k < R; ++k)
-      if (tb + k < te) wide_copy<FMT, MT, NT, BLOCK, WM>(p, ring + k * S::BYTES, tb + k, wv, lane, L, sa_ring);
+      if (tb + k < te) wide_copy<FMT, MT, NT, BLOCK>(p, ring + k * S::BYTES, tb + k, wv, lane, L, sa_ring);
     wide_wait<C, R - 1>((int)(te - 1 - tb < R - 1 ? te - 1 - tb : R - 1), wv < S::SW);
     wide_barrier();
-    WideRegs<MTW, NT, BLOCK> x0, x1;
-    wide_read<FMT, MT, NT, BLOCK, WM>(ring, sa_ring + ((tb >> 2) % 3) * S::RING_ENTRY, (int)(tb & 3), wv, lane, q, r,
+    WideRegs<MT, NT, BLOCK> x0, x1;
+    wide_read<FMT, MT, NT, BLOCK>(ring, sa_ring + ((tb >> 2) % 3) * S::RING_ENTRY, (int)(tb & 3), wv, lane, q, r,
                                   x0);
     if (BLOCK) x0.sbv = sb_stage[0];
 
@@ -465,14 +440,14 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
         wide_wait<C, R - 2>((int)later, wv < S::SW);                                                  \
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                          \
         wide_barrier();                                                                             \
-        if (tt + R < te) wide_copy<FMT, MT, NT, BLOCK, WM>(p, ring + ((I_) % R) * S::BYTES, tt + R, wv, lane, L, sa_ring); \
+        if (tt + R < te) wide_copy<FMT, MT, NT, BLOCK>(p, ring + ((I_) % R) * S::BYTES, tt + R, wv, lane, L, sa_ring); \
       }                                                                                             \
-      wide_read<FMT, MT, NT, BLOCK, WM>(ring + ((I_ + 1) % R) * S::BYTES,                           \
+      wide_read<FMT, MT, NT, BLOCK>(ring + ((I_ + 1) % R) * S::BYTES,                           \
                                     sa_ring + (((tt + 1) >> 2) % 3) * S::RING_ENTRY,            \
                                 (int)((tt + 1) & 3), wv, lane, q, r, NXT_);                         \
       if (BLOCK) NXT_.sbv = sb_stage[(tt + 1 < te ? tt + 1 : tt) - tb];                             \
-      wide_mfma<FMT, MTW, NT, BLOCK>(CUR_, acc);                                                    \
-      wide_interleave<FMT, MTW, NT, BLOCK>();                                                       \
+      wide_mfma<FMT, MT, NT, BLOCK>(CUR_, acc);                                                    \
+      wide_interleave<FMT, MT, NT, BLOCK>();                                                       \
     }                                                                                               \
   }
 
@@ -513,8 +488,8 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-      for (int i = 0; i < MTW; ++i) {
-        const int f = (wm * MTW + i) * (4 * NT) + wn * NT + n;
+      for (int i = 0; i < MT; ++i) {
+        const int f = i * (4 * NT) + wv * NT + n;
         *reinterpret_cast<float4*>(pdst + (f * 64 + lane) * 4) =
             float4{acc[i][n][0], acc[i][n][1], acc[i][n][2], acc[i][n][3]};
       }
@@ -525,10 +500,10 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
-    for (int i = 0; i < MTW; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        tile[(16 * (wm * MTW + i) + 4 * q + e) * ST + 16 * (wn * NT + n) + r] = acc[i][n][e];
+        tile[(16 * i + 4 * q + e) * ST + 16 * (wv * NT + n) + r] = acc[i][n][e];
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   const int64_t col0 = nb * TW;
   // Tiles whose columns all lie inside N (rows are checked per piece) take batched
@@ -607,10 +582,10 @@ constexpr int kWideMaxExperts = (int)kWideGroupedMaxExperts;
 
 // The grouped variant runs two workgroups per CU (at most 256 registers per lane and
 // half the LDS each).
-template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED, int WM = 1>
-__global__ __launch_bounds__(256 * WM, GROUPED ? 2 : 1) void gemm_wide_kernel(GemmParams p, WideGrid g) {
-  static_assert(WM == 1 || !GROUPED, "the grouped variant runs four waves");
-  using S = WideSlot<MT, NT, BLOCK, WM>;
+template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED>
+struct WideKernel<FMT, MT, NT, BLOCK, GROUPED, 1> {
+static __device__ __forceinline__ void run(const GemmParams& p, const WideGrid& g) {
+  using S = WideSlot<MT, NT, BLOCK>;
   constexpr int BM = 16 * MT;
   // the stage ring (dense: the LDS budget of one workgroup per CU; grouped: two slots);
   // after the last stage it holds the output tile of the epilogue
@@ -624,36 +599,34 @@ __global__ __launch_bounds__(256 * WM, GROUPED ? 2 : 1) void gemm_wide_kernel(Ge
 
   if (!GROUPED) {
     // XCD-aware remap of the linear workgroup id: the m-blocks sharing a weight
-    // slice run consecutively on one XCD (workgroup L runs on XCD L % 8)
-    const int64_t G = gridDim.x, Lid = blockIdx.x;
-    const int64_t xcd = Lid & 7, per = G >> 3, extra = G & 7;
-    const int64_t logical = xcd * per + (xcd < extra ? xcd : extra) + (Lid >> 3);
+    // slice run consecutively on one XCD
+    const int64_t logical = wide_logical(blockIdx.x, gridDim.x);
     constexpr int TW = 64 * NT;
-    // (the two waves of an n-group share its row: they copy the same scales to it)
-    float* const sbw = sb_lds + (BLOCK ? (wv & 3) * kWideBlockStages : 0);
+    float* const sbw = sb_lds + (BLOCK ? wv * kWideBlockStages : 0);
     const uint8_t* const sw = static_cast<const uint8_t*>(p.sw);
     if (g.rem_tiles == 0) {
       const int64_t local = logical % g.tiles, split = logical / g.tiles;
-      const int64_t tile = g.tile0 + local;
-      const int64_t mb = tile % g.mblocks, nb = tile / g.mblocks;
+      int64_t mb, nb;
+      wide_coords(local, g.mblocks, g.nblocks, g.group_m, mb, nb);
       // split partials: the tile's fragment-ordered block, [split][tile][BM x TW]
       float* const pdst = p.S == 1 ? nullptr : p.partial + (split * g.tiles + local) * BM * TW;
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED, WM>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, split, pdst, ring,
+      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, split, pdst, ring,
                                                  sa_ring, sbw, t, lane, wv, r, q);
       return;
     }
     // one-launch hybrid: the whole-K tile, then the remainder unit (if any)
     if (logical < g.tiles) {
-      const int64_t mb = logical % g.mblocks, nb = logical / g.mblocks;
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED, WM>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, 0, nullptr, ring,
+      int64_t mb, nb;
+      wide_coords(logical, g.mblocks, g.nblocks, g.group_m, mb, nb);
+      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, 0, nullptr, ring,
                                                  sa_ring, sbw, t, lane, wv, r, q);
     }
     if (logical < g.rem_tiles * g.S2) {
       const int64_t local = logical % g.rem_tiles, split = logical / g.rem_tiles;
-      const int64_t tile = g.rem_tile0 + local;
-      const int64_t mb = tile % g.mblocks, nb = tile / g.mblocks;
+      int64_t mb, nb;
+      wide_coords(g.rem_tile0 + local, g.mblocks, g.nblocks, g.group_m, mb, nb);
       __syncthreads();  // the first tile's epilogue reads of the ring are done
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED, WM>(p, g.kt2, mb * BM, p.M, p.w, sw, nb, split,
+      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt2, mb * BM, p.M, p.w, sw, nb, split,
                                                  p.partial + (split * g.rem_tiles + local) * BM * TW, ring, sa_ring,
                                                  sbw, t, lane, wv, r, q);
     }
@@ -718,37 +691,41 @@ __global__ __launch_bounds__(256 * WM, GROUPED ? 2 : 1) void gemm_wide_kernel(Ge
     // a 128-row block with at most 64 routed rows (an expert's last block) runs the
     // 64-row tile path in the same ring: half the activation copies and MFMAs
     if (MT == 8 && __builtin_amdgcn_readfirstlane((int)(rhi - rb)) <= 64)
-      wide_tile<FMT, (MT == 8 ? 4 : MT), NT, BLOCK, GROUPED, 1>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr,
+      wide_tile<FMT, (MT == 8 ? 4 : MT), NT, BLOCK, GROUPED>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr,
                                                              ring, sa_ring, sb_lds, t, lane, wv, r, q);
     else
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED, 1>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr, ring, sa_ring,
+      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr, ring, sa_ring,
                                              sb_lds, t, lane, wv, r, q);
     __syncthreads();  // the epilogue's LDS reads are done before the next tile's copies
   }
 }
+};
 
 // Sum the split partials of output tiles [tile0, tile0 + tiles) in split order, then the
 // output rounding (out_bits: alpha, format, bias; the split-K reduce's arithmetic).  The
 // partials are fragment-ordered tile blocks, [split][tile - tile0][BM x TW]: fragment f =
 // m-tile * (TW / 16) + n-tile of a block is 64 lanes x 4 floats, lane (q, r) holding rows
-// 4 q .. 4 q + 3 of column r.  One thread per (tile, fragment, lane): its S float4 loads
-// are contiguous across the wave, and each of its four rows gets one 2-byte store (sixteen
-// lanes cover 32 contiguous bytes of a row).
+// 4 q .. 4 q + 3 of column r (four-wave tiles) or columns 4 q .. 4 q + 3 of row r (cols4,
+// the 2 x 2-wave tiles).  One thread per (tile, fragment, lane): its S float4 loads are
+// contiguous across the wave; its four results are one 2-byte store per row, or one 8-byte
+// store of a row (32 contiguous bytes of it over the fragment's four q).
 #ifndef MXL_WIDE_MX_DENSE_ONLY
 __global__ __launch_bounds__(256) void wide_tile_reduce_kernel(const float* __restrict__ partial,
                                                                const uint16_t* __restrict__ bias,
                                                                uint16_t* __restrict__ out, int64_t M, int64_t N,
-                                                               int64_t ldc, int64_t mblocks, int64_t tile0,
-                                                               int64_t tiles, int S, int BM, int TW, float alpha,
-                                                               int f16) {
+                                                               int64_t ldc, WideGrid g, int64_t tile0,
+                                                               int64_t tiles, int S, int BM, int TW, int cols4,
+                                                               float alpha, int f16) {
   const int64_t per_tile = (int64_t)BM * TW / 4;  // float4 items of a tile block
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= tiles * per_tile) return;
   const int64_t local = id / per_tile;
   const int item = (int)(id - local * per_tile), f = item >> 6, lane = item & 63;
   const int nts = TW / 16;
-  const int64_t tile = tile0 + local, mb = tile % mblocks, nb = tile / mblocks;
-  const int64_t row0 = mb * BM + 16 * (f / nts) + 4 * (lane >> 4), col = nb * TW + 16 * (f % nts) + (lane & 15);
+  int64_t mb, nb;
+  wide_coords(tile0 + local, g.mblocks, g.nblocks, g.group_m, mb, nb);
+  const int step = cols4 ? (lane & 15) : 4 * (lane >> 4), across = cols4 ? 4 * (lane >> 4) : (lane & 15);
+  const int64_t row0 = mb * BM + 16 * (f / nts) + step, col = nb * TW + 16 * (f % nts) + across;
   if (row0 >= M || col >= N) return;
   const float4* src = reinterpret_cast<const float4*>(partial) + local * per_tile + item;
   const int64_t stride = tiles * per_tile;  // float4s per split
@@ -766,6 +743,21 @@ __global__ __launch_bounds__(256) void wide_tile_reduce_kernel(const float* __re
   }
   const float a4[4] = {acc.x, acc.y, acc.z, acc.w};
   const bool b = bias != nullptr;
+  if (cols4) {
+    uint16_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      h[e] = out_bits(a4[e], alpha, f16, b, b ? bias[col + e < N ? col + e : N - 1] : (uint16_t)0);
+    uint16_t* dst = out + row0 * ldc + col;
+    if (col + 4 <= N && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0) {
+      *reinterpret_cast<uint2*>(dst) = uint2{h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < N) dst[e] = h[e];
+    }
+    return;
+  }
   const uint16_t bv = b ? bias[col] : (uint16_t)0;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
@@ -881,6 +873,93 @@ WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptio
   return best;
 }
 
+// ---- 2 x 2-wave tiles
+//
+// Time model, fitted to a sweep of every tile and split over 184 dense shapes (M 17..2048, N
+// 256..18432, K 512..17408, MXFP8, MXFP6 and block-FP8 weights rotated out of the caches): a launch
+// costs its fixed time, the stages of the fullest CU, its operands from HBM and its output, which
+// nothing overlaps in the last round.  Its pick runs within 0.9 % of the best of them on average
+// (the farthest: 722 x 11264 x 896 21.0 us against 18.1, 561 x 1792 x 17408 38.4 against 32.9).
+struct TileCost {
+  int MT, NT, resident;   // tile, workgroups per CU
+  double fixed, stage;    // us: of the launch, of a K128 stage on one CU
+  double quarter;         // us: of a K128 stage of a quarter tile (0: no quarters)
+};
+constexpr TileCost kTileCosts[] = {{16, 4, 1, 4.9, 1.07, 0.402}, {8, 4, 1, 4.3, 0.693, 0.300},
+                                   {8, 2, 2, 4.4, 0.402, 0.207}, {8, 1, 2, 3.8, 0.289, 0},
+                                   {4, 2, 2, 3.7, 0.300, 0},     {4, 1, 4, 3.4, 0.207, 0}};
+// a block-FP8 stage against an MX one: a workgroup waits for its own folds, two take turns
+constexpr double kTileBlockAlone = 1.06, kTileBlockShared = 0.874;
+constexpr double kTileGap = 0.5;                  // a further round's start on a CU, us
+constexpr double kTileReduce = 3.2;               // the split reduce's launch, us
+constexpr double kTileBytesPerUs = 10.6e6, kTileOutBytesPerUs = 2.3e6, kTilePartialBytesPerUs = 6.1e6;
+// the few tiles of a hybrid's remainder: their partials stay in the caches
+constexpr double kTileRemainderBytesPerUs = 8.9e6;
+
+// Tiles of a partly filled last round that run as four quarters each, so that their K walk ends
+// sooner: where the quarters' stages on the fullest CU are clearly fewer than the tile's (W6A8
+// 1024 x 17408 x 5120 in 256 x 256 tiles, 16 past a full round: 116.6 to 95.2 us; block-FP8 512 x
+// 18432 x 2560 in 128 x 128, 64 past 512: 44.2 to 37.1).  After at least one full round of
+// resident workgroups: with fewer tiles the hybrid below splits the remainder in K.
+static int64_t wide_tail(const TileCost& t, int64_t tiles, int64_t cus) {
+  const int64_t rem = tiles % cus;
+  if (t.quarter == 0 || tiles <= t.resident * cus || rem == 0) return 0;
+  return (double)((4 * rem + cus - 1) / cus) * t.quarter < 0.9 * t.stage ? rem : 0;
+}
+
+bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
+  // 32-bit operand offsets
+  return M * K < (int64_t(1) << 32) && ((N + 15) / 16) * ((K + kTileK - 1) / kTileK) < (1 << 24) &&
+         (!block || K <= int64_t(128) * kWideBlockStages);
+}
+
+// Tile, split and hybrid of the 2 x 2-wave kernels by the time model.
+WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool block) {
+  const int64_t KT = (K + kTileK - 1) / kTileK, T = (K + 127) / 128, cus = cu_count();
+  const double weights = (double)N * K * (fmt == kE4M3 ? 1.0 : 0.75) + (double)N * K / 32;
+  const double in = (weights + (double)M * K) / kTileBytesPerUs;
+  const double out = 2.0 * M * N / kTileOutBytesPerUs;
+  WideConfig best{2, 1, KT};
+  double best_us = 1e300;
+  for (const TileCost& t : kTileCosts) {
+    if (block && t.NT == 4) continue;  // (not instantiated)
+    const int64_t tiles = ((M + 16 * t.MT - 1) / (16 * t.MT)) * ((N + 64 * t.NT - 1) / (64 * t.NT));
+    // `n` workgroups of `stages` stages on the fullest CU
+    auto work = [&](int64_t n, int64_t stages) -> double {
+      const double factor = !block ? 1.0 : n % t.resident == 1 ? kTileBlockAlone : kTileBlockShared;
+      return n * stages * t.stage * factor + ((n + t.resident - 1) / t.resident - 1) * kTileGap;
+    };
+    auto take = [&](double us, const WideConfig& c) {
+      if (us >= best_us) return;
+      best_us = us;
+      best = c;
+      best.MT = t.MT;
+    };
+    for (int64_t s = 1; s <= KT && s <= 16; ++s) {
+      const int64_t per = (KT + s - 1) / s;
+      if ((KT + per - 1) / per != s) continue;
+      const int64_t stages = per * 4 < T ? per * 4 : T, n = (tiles * s + cus - 1) / cus;
+      const int64_t tail = s == 1 ? wide_tail(t, tiles, cus) : 0;
+      double us = t.fixed + in;
+      if (tail) us += work(n - 1, stages) + (4 * tail + cus - 1) / cus * stages * t.quarter + kTileGap;
+      else us += work(n, stages);
+      if (s == 1) us += out;
+      else us += kTileReduce + ((double)M * N * 8 * s + 2.0 * M * N) / kTilePartialBytesPerUs;
+      take(us, WideConfig{t.NT, (int)s, per});
+    }
+    // the hybrid after one full round only (after two it measured within 6 % of whole-K either
+    // way): block-FP8 256 x 18432 x 2560 27.5 us against 30.5 whole-K, W6A8 256 x 17408 x 5120 40.2
+    // against 54.1.  (Quarters for the remainder would take 24.3 and 40.3 there.)
+    WideConfig h{t.NT, 1, KT};
+    if (t.MT == 8 && t.NT == 2 && wide_hybrid(tiles, KT, cus, h) && h.dp_tiles == cus)
+      take(t.fixed + in + work(1, T) + h.kt2 * 4 * t.stage * (block ? kTileBlockShared : 1.0) + kTileReduce +
+               (double)(tiles - cus) * 128 * 128 * 8 * h.S2 / kTileRemainderBytesPerUs,
+           h);
+  }
+  best.WM = 2;
+  return best;
+}
+
 int64_t wide_workspace_bytes(const WideConfig& c, int64_t M, int64_t N) {
   // fragment-ordered partial blocks of whole tiles (padding rows and columns included)
   const int64_t bm = 16 * c.MT;
@@ -897,33 +976,14 @@ template <int FMT, int MT, bool BLOCK, bool GROUPED>
 static hipError_t launch_wide_mt(const WideConfig& c, const GemmParams& p, const WideGrid& g, int64_t grid,
                                  hipStream_t s) {
   const dim3 gr((unsigned)grid), blk(256);
-  if (c.WM == 2) {  // eight waves: dense 128-row tiles
-    if constexpr (GROUPED || MT != 8) {
-      return hipErrorInvalidValue;
-    } else {
-      const dim3 blk8(512);
-      if (c.NT == 4) {
-        // block-FP8 with four n-tiles per wave does not fit two waves' registers per SIMD
-        if constexpr (BLOCK) return hipErrorInvalidValue;
-        else hipLaunchKernelGGL((gemm_wide_kernel<FMT, 8, 4, false, false, 2>), gr, blk8, 0, s, p, g);
-      } else if (c.NT == 2) {
-        hipLaunchKernelGGL((gemm_wide_kernel<FMT, 8, 2, BLOCK, false, 2>), gr, blk8, 0, s, p, g);
-      } else if (c.NT == 1) {
-        hipLaunchKernelGGL((gemm_wide_kernel<FMT, 8, 1, BLOCK, false, 2>), gr, blk8, 0, s, p, g);
-      } else {
-        return hipErrorInvalidValue;
-      }
-      return hipGetLastError();
-    }
-  }
   if (c.NT == 4) {
     if constexpr (GROUPED) return hipErrorInvalidValue;  // the grouped variant runs NT <= 2 (LDS)
-    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 4, BLOCK, GROUPED>), gr, blk, 0, s, p, g);
+    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 4, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
   } else if (c.NT == 2) {
-    hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 2, BLOCK, GROUPED>), gr, blk, 0, s, p, g);
+    hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 2, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
   } else if (c.NT == 1) {
     if constexpr (MT == 4) return hipErrorInvalidValue;  // 64 x 64 tiles are not instantiated
-    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 1, BLOCK, GROUPED>), gr, blk, 0, s, p, g);
+    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 1, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
   } else {
     return hipErrorInvalidValue;
   }
@@ -972,9 +1032,13 @@ hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const Gemm
     return hipErrorInvalidValue;
   }
   g.mblocks = (p.M + bm - 1) / bm;
-  g.tile0 = 0;
   g.tiles = g.mblocks * g.nblocks;
+  // four-wave tiles: all m-blocks of a weight slice together; 2 x 2-wave tiles: about 1024
+  // rows by the n-blocks an XCD's CUs reach at a time, so that both operands' slices stay
+  // few (M = 4096, N = 17408, K = 5120: 1024 rows 305 us, 2048 rows 329, all 302)
+  g.group_m = c.WM == 2 && g.mblocks * bm > 1024 ? 1024 / bm : g.mblocks;
   auto dense = [&](const GemmParams& q, const WideGrid& gg, int64_t n) -> hipError_t {
+    if (c.WM == 2) return launch_wide_tiles(fmt, block, c, q, gg, n, s);
     if (block) return fmt == kE4M3 ? launch_wide_fmt<kE4M3, true, false>(c, q, gg, n, s) : hipErrorInvalidValue;
     return launch_wide_mx_dense(fmt, c, q, gg, n, s);
   };
@@ -982,19 +1046,28 @@ hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const Gemm
   auto tile_reduce = [&](int64_t tile0, int64_t tiles, int S) -> hipError_t {
     const int64_t items = tiles * bm * tw / 4;
     wide_tile_reduce_kernel<<<dim3((unsigned)((items + 255) / 256)), 256, 0, s>>>(
-        p.partial, p.bias, p.out, p.M, p.N, p.ldc, g.mblocks, tile0, tiles, S, (int)bm, (int)tw, p.alpha, p.out_f16);
+        p.partial, p.bias, p.out, p.M, p.N, p.ldc, g, tile0, tiles, S, (int)bm, (int)tw, c.WM == 2, p.alpha,
+        p.out_f16);
     return hipGetLastError();
   };
   if (c.dp_tiles <= 0 || c.dp_tiles >= g.tiles) {
     // every tile in one launch, split in K into fragment-ordered partials when S > 1
-    const hipError_t e = dense(p, g, g.tiles * c.S);
+    g.tail0 = g.tiles * c.S;
+    int64_t units = g.tail0;
+    if (c.WM == 2 && c.S == 1) {
+      for (const TileCost& t : kTileCosts)
+        if (t.MT == c.MT && t.NT == c.NT) g.tail0 = g.tiles - wide_tail(t, g.tiles, cu_count());
+      units = g.tail0 + 4 * (g.tiles - g.tail0);
+    }
+    const hipError_t e = dense(p, g, units);
     if (e != hipSuccess || p.S == 1) return e;
     return tile_reduce(0, g.tiles, p.S);
   }
-  // hybrid, one launch: workgroup L runs whole-K tile L (full rounds, bf16 out) and then
-  // unit L of the remainder, split in K into compact partials (p.partial); their reduce
-  // follows.  (With more than one full round some units run in later rounds' workgroups;
-  // the last round still ends one unit after its tiles.)
+  // hybrid, one launch: whole-K tiles (full rounds, bf16 out) and the remainder's units, split
+  // in K into compact partials (p.partial); their reduce follows.  Four-wave: workgroup L runs
+  // tile L and then unit L (with more than one full round some units run in later rounds'
+  // workgroups; the last round still ends one unit after its tiles).  2 x 2-wave: the units are
+  // workgroups of their own beside the last round's.
   GemmParams q = p;
   q.S = 1;
   WideGrid gd = g;
@@ -1004,7 +1077,8 @@ hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const Gemm
   gd.kt2 = c.kt2;
   gd.S2 = c.S2;
   const int64_t units = gd.rem_tiles * c.S2;
-  hipError_t e = dense(q, gd, c.dp_tiles > units ? c.dp_tiles : units);
+  gd.tail0 = c.dp_tiles;
+  hipError_t e = dense(q, gd, c.WM == 2 ? c.dp_tiles + units : c.dp_tiles > units ? c.dp_tiles : units);
   if (e != hipSuccess) return e;
   return tile_reduce(gd.rem_tile0, gd.rem_tiles, c.S2);
 }

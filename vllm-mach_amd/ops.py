@@ -130,7 +130,8 @@ def tuning(kernel: int = KERNEL_AUTO, splits: int = 0, tile_n: int = 0, tile_m: 
     """Force the GEMM kernel / wide tile / K split of every GEMM call inside the block
     (``mxl_gemm_options``; the reference's tactic and splits overrides,
     src/vllm_mach/mxfp8/native_backend.py:29).  Grouped GEMMs read ``kernel`` (their
-    schedule) and ``tile_m``; ``waves`` (4 or 8) picks the wide MX kernel's workgroup size.
+    schedule) and ``tile_m``; ``waves`` (4 or 8) picks the wide kernel's waves per CU (one workgroup
+    of four side by side, or two of 2 x 2).
     For tuning runs and tests."""
     global _tuning
     old = _tuning
