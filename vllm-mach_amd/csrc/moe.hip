@@ -10,7 +10,8 @@
 // workgroup when the histograms fit in LDS), then a pass that
 // ranks each route inside its chunk (a ballot match of the expert id's bits inside the
 // wavefront plus an LDS prefix over the chunk's 16 wavefronts) and scatters.  A single chunk
-// (decode-sized steps) runs all three in one workgroup.
+// (decode-sized steps) runs all three in one workgroup; up to 32 chunks run them in one launch
+// that counts in every workgroup.
 //
 // Combine: out[t, h] = bf16(sum_k y[inverse[t*topk + k], h] * w[t, k]),
 // each product rounded to binary32 and added in ascending k from zero.
@@ -237,179 +238,45 @@ __global__ __launch_bounds__(kChunk) void route_single_kernel(const int32_t* __r
   single_chunk_sort(t < R ? ids[t] : -1, R, E, expert_offsets, sorted_routes, inverse, whist, tot);
 }
 
-// ------------------------------------------------------------------ router
-//
-// softmax -> top-k -> (renormalize) from router logits, the selection of vLLM's fused
-// top-k softmax that the reference's MoE layer runs before its experts (select_experts;
-// src/vllm_mach/mxfp6/moe.py:142-152 fuses it into qwen35_router_quant_out): the k largest
-// logits of a token (softmax is increasing, so they are its k largest probabilities), ties
-// to the lower expert index, weights exp(x - max) / sum, the sum over the k selected
-// (renormalize) or over every expert.  One wavefront per token, the token's logits spread
-// over its lanes (expert i at lane i % 64, slot i / 64); each of the k rounds takes the
-// wavefront maximum of (order key, lower index) over the logits not yet taken.
-
-constexpr int kRouterSlots = kSingleMaxExperts / 64;  // logits per lane: E <= 1024
-constexpr int kRouterMaxTopk = 64;
-
-// Binary32 as an unsigned key in value order (-0 read as +0, so equal values tie; NaNs
-// order outside the finite values by sign).
-__device__ __forceinline__ uint32_t order_key(float x) {
-  uint32_t u = f2u(x);
-  if (u == 0x80000000u) u = 0u;
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float key_value(uint32_t k) { return u2f((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k); }
-
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m, 64);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m, 64);
-    const uint64_t o = ((uint64_t)hi << 32) | lo;
-    v = o > v ? o : v;
-  }
-  return v;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);
-  return v;
-}
-
-// Route token t with the calling wavefront: ids / weights [t * topk + r] for r < topk;
-// returns the lane's id (lane r < topk holds selection r, other lanes -1).
-template <bool BF16>
-__device__ __forceinline__ int32_t route_token(const void* __restrict__ logits, int64_t t, int E, int topk,
-                                               bool renorm, int lane, int32_t* __restrict__ ids,
-                                               float* __restrict__ weights) {
-  uint32_t key[kRouterSlots];
-#pragma unroll
-  for (int j = 0; j < kRouterSlots; ++j) {
-    const int i = lane + 64 * j;
-    float x = 0.0f;
-    if (i < E) x = BF16 ? bf16_to_f32(static_cast<const uint16_t*>(logits)[t * E + i])
-                        : static_cast<const float*>(logits)[t * E + i];
-    key[j] = i < E ? order_key(x) : 0u;
-  }
-  uint32_t taken = 0u;
-  float my_x = 0.0f;
-  int32_t my_id = -1;
-  float top = 0.0f;
-  for (int r = 0; r < topk; ++r) {
-    uint64_t best = 0;  // (key, ~index): the larger key, then the lower index
-#pragma unroll
-    for (int j = 0; j < kRouterSlots; ++j) {
-      const int i = lane + 64 * j;
-      if (i < E && !((taken >> j) & 1u)) {
-        const uint64_t c = ((uint64_t)key[j] << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)i);
-        best = c > best ? c : best;
-      }
-    }
-    best = wave_max_u64(best);
-    const int idx = (int)(0xFFFFFFFFu - (uint32_t)best);
-    const float x = key_value((uint32_t)(best >> 32));
-    if ((idx & 63) == lane) taken |= 1u << (idx >> 6);
-    if (r == 0) top = x;
-    if (lane == r) {
-      my_x = x;
-      my_id = idx;
-    }
-  }
-  const float e = lane < topk ? mx_exp(my_x - top) : 0.0f;
-  float denom;
-  if (renorm) {
-    denom = wave_sum(e);
-  } else {
-    float part = 0.0f;
-#pragma unroll
-    for (int j = 0; j < kRouterSlots; ++j)
-      if (lane + 64 * j < E) part = part + mx_exp(key_value(key[j]) - top);
-    denom = wave_sum(part);
-  }
-  if (lane < topk) {
-    ids[t * topk + lane] = my_id;
-    weights[t * topk + lane] = e / denom;
-  }
-  return my_id;
-}
-
-// T * topk <= 1024 routes and E <= 1024: routing and the token sort in one workgroup.
-template <bool BF16>
-__global__ __launch_bounds__(kChunk) void router_single_kernel(const void* __restrict__ logits, int64_t T, int E,
-                                                              int topk, int renorm, int32_t* __restrict__ ids,
-                                                              float* __restrict__ weights,
-                                                              int64_t* __restrict__ expert_offsets,
-                                                              int32_t* __restrict__ sorted_routes,
-                                                              int32_t* __restrict__ inverse) {
-  __shared__ int32_t whist[(kChunk / 64) * kSingleMaxExperts];
-  __shared__ int32_t tot[2][kSingleMaxExperts];
-  __shared__ int32_t sids[kChunk];
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  for (int64_t tok = w; tok < T; tok += kChunk / 64) {
-    const int32_t id = route_token<BF16>(logits, tok, E, topk, renorm != 0, lane, ids, weights);
-    if (lane < topk) sids[tok * topk + lane] = id;
-  }
-  __syncthreads();
-  const int64_t R = T * topk;
-  single_chunk_sort(t < R ? sids[t] : -1, R, E, expert_offsets, sorted_routes, inverse, whist, tot);
-}
-
-// Chunk c of 1024 routes = 1024 / topk whole tokens (topk divides 1024): route them and
-// count the chunk's routes per expert (the histogram the scatter's chunk bases come from).
-template <bool BF16>
-__global__ __launch_bounds__(kChunk) void router_hist_kernel(const void* __restrict__ logits, int64_t T, int E,
-                                                            int topk, int renorm, int32_t* __restrict__ ids,
-                                                            float* __restrict__ weights,
-                                                            int32_t* __restrict__ chunk_counts) {
-  __shared__ int32_t hist[kSingleMaxExperts];
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int64_t c = blockIdx.x, per = kChunk / topk;
-  for (int e = t; e < E; e += kChunk) hist[e] = 0;
-  __syncthreads();
-  for (int64_t k = w; k < per; k += kChunk / 64) {
-    const int64_t tok = c * per + k;
-    if (tok >= T) break;
-    const int32_t id = route_token<BF16>(logits, tok, E, topk, renorm != 0, lane, ids, weights);
-    if (lane < topk) atomicAdd(&hist[id], 1);
-  }
-  __syncthreads();
-  for (int e = t; e < E; e += kChunk) chunk_counts[c * E + e] = hist[e];
-}
-
-// Every chunk's scatter from the chunk histograms (C x E <= kCountScanMaxEntries,
-// E <= 1024): the workgroup sums the histograms of the chunks before its own (its chunk
-// bases) and of all chunks (the expert totals, scanned into the offsets, which workgroup 0
-// writes), then ranks and scatters its routes as route_scatter_kernel does.
-__global__ __launch_bounds__(kChunk) void route_scan_scatter_kernel(const int32_t* __restrict__ ids, int64_t R,
-                                                                   int64_t C, int E,
-                                                                   const int32_t* __restrict__ chunk_counts,
-                                                                   int64_t* __restrict__ expert_offsets,
-                                                                   int32_t* __restrict__ sorted_routes,
-                                                                   int32_t* __restrict__ inverse) {
+// 2 .. kSortMaxChunks chunks in one launch (E <= 1024): every workgroup counts all routes for
+// itself, those of the chunks before its own apart from the rest (one LDS atomic per route and
+// workgroup), scans the totals into the offsets, which workgroup 0 writes, and ranks and
+// scatters its chunk as route_scatter_kernel does.  Repeating the counts costs less than the
+// launches that share them (16384 routes of 256 experts: 6.7 us against 9.2 for
+// route_count_scan_kernel and route_scatter_kernel), up to 32 chunks, where a thread counts 32.
+constexpr int kSortMaxChunks = 32;
+__global__ __launch_bounds__(kChunk) void route_sort_kernel(const int32_t* __restrict__ ids, int64_t R, int C, int E,
+                                                           int64_t* __restrict__ expert_offsets,
+                                                           int32_t* __restrict__ sorted_routes,
+                                                           int32_t* __restrict__ inverse) {
   constexpr int W = kChunk / 64;
-  __shared__ int32_t whist[W * kSingleMaxExperts];
-  __shared__ int32_t base[kSingleMaxExperts];
-  __shared__ int32_t tot[2][kSingleMaxExperts];
-  const int64_t c = blockIdx.x;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  for (int x = t; x < E; x += kChunk) {
-    int32_t before = 0, all = 0;
-    for (int64_t cc = 0; cc < C; ++cc) {
-      const int32_t n = chunk_counts[cc * E + x];
-      if (cc < c) before += n;
-      all += n;
+  extern __shared__ int32_t lds[];
+  int32_t* const whist = lds;                                           // [W][E]
+  int32_t *const before = whist + W * E, *const rest = before + E;      // routes of earlier chunks, of the others
+  int32_t* const tot[2] = {rest + E, rest + 2 * E};
+  const int c = blockIdx.x, t = threadIdx.x, w = t >> 6, lane = t & 63;
+  for (int i = t; i < W * E + 2 * E; i += kChunk) lds[i] = 0;
+  __syncthreads();
+  int32_t e = -1;
+  for (int c0 = 0; c0 < C; c0 += 8) {
+    int32_t x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t r = (int64_t)(c0 + k) * kChunk + t;
+      x[k] = r < R ? ids[r] : -1;
     }
-    base[x] = before;
-    tot[0][x] = all;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (c0 + k == c) e = x[k];
+      if (x[k] >= 0 && x[k] < E) atomicAdd((c0 + k < c ? before : rest) + x[k], 1);
+    }
   }
-  for (int i = t; i < W * E; i += kChunk) whist[i] = 0;
-  const int64_t r = c * kChunk + t;
-  const int32_t e = r < R ? ids[r] : -1;
+  const int64_t r = (int64_t)c * kChunk + t;
   const bool valid = e >= 0 && e < E;
   const int rank = same_expert_rank(valid ? e : E, E, lane);
-  __syncthreads();
   if (valid) atomicAdd(&whist[w * E + e], 1);
+  __syncthreads();
+  for (int x = t; x < E; x += kChunk) tot[0][x] = before[x] + rest[x];
   int src = 0;  // inclusive scan of the totals (ping-pong)
   for (int d = 1; d < E; d <<= 1) {
     __syncthreads();
@@ -426,7 +293,7 @@ __global__ __launch_bounds__(kChunk) void route_scan_scatter_kernel(const int32_
     if (t == 0) expert_offsets[0] = 0;
   }
   for (int x = t; x < E; x += kChunk) {
-    int32_t run = 0;
+    int32_t run = before[x] + (x > 0 ? tot[src][x - 1] : 0);
     for (int v = 0; v < W; ++v) {
       const int32_t n = whist[v * E + x];
       whist[v * E + x] = run;
@@ -439,19 +306,155 @@ __global__ __launch_bounds__(kChunk) void route_scan_scatter_kernel(const int32_
     inverse[r] = -1;
     return;
   }
-  const int64_t pos = (e > 0 ? tot[src][e - 1] : 0) + base[e] + whist[w * E + e] + rank;
+  const int32_t pos = whist[w * E + e] + rank;
   sorted_routes[pos] = (int32_t)r;
-  inverse[r] = (int32_t)pos;
+  inverse[r] = pos;
 }
 
-// Routing only (shapes the fused schedules above do not take): ids and weights, sorted by
-// mxl_moe_route afterwards.
-template <bool BF16>
+// ------------------------------------------------------------------ router
+//
+// softmax -> top-k -> (renormalize) from router logits, the selection of vLLM's fused
+// top-k softmax that the reference's MoE layer runs before its experts (select_experts;
+// src/vllm_mach/mxfp6/moe.py:142-152 fuses it into qwen35_router_quant_out): the k largest
+// logits of a token (softmax is increasing, so they are its k largest probabilities), ties
+// to the lower expert index, weights exp(x - max) / sum, the sum over the k selected
+// (renormalize) or over every expert.  One wavefront per token, the token's logits spread
+// over its lanes (expert i at lane i % 64, slot i / 64; NS slots, 4 for up to 256 experts); each
+// of the k rounds takes the wavefront maximum of the keys not yet taken by DPP moves, and the
+// lowest expert that holds it from one ballot per slot.  The rounds are a serial chain of some
+// 30 instructions each, so the routing is spread over the chip, one wavefront per SIMD, whenever
+// one workgroup's wavefronts would have to take several tokens each.  (With 16 slots of 64-bit
+// keys, exchanged over the LDS crossbar, and all tokens of a chunk of 1024 routes in one
+// workgroup: 64 tokens of 256 experts, top 8, with the sort 38.5 us, now 8.1; 2048 tokens 78,
+// now 11.5.)
+
+constexpr int kRouterSlots = kSingleMaxExperts / 64;  // logits per lane: E <= 1024
+constexpr int kRouterMaxTopk = 64;
+
+// Binary32 as an unsigned key in value order (-0 read as +0, so equal values tie; NaNs
+// order outside the finite values by sign).
+__device__ __forceinline__ uint32_t order_key(float x) {
+  uint32_t u = f2u(x);
+  if (u == 0x80000000u) u = 0u;
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float key_value(uint32_t k) { return u2f((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k); }
+
+// The wavefront's largest value, in every lane: an inclusive maximum along the lanes (rows of
+// 16, then across rows), read from lane 63.  Lanes without a source keep 0.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#define MXL_DPP_MAX(CTRL_, ROWS_)                                                              \
+  {                                                                                            \
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL_, ROWS_, 0xf, false); \
+    v = o > v ? o : v;                                                                         \
+  }
+  MXL_DPP_MAX(0x111, 0xf)  // row_shr:1, 2, 4, 8
+  MXL_DPP_MAX(0x112, 0xf)
+  MXL_DPP_MAX(0x114, 0xf)
+  MXL_DPP_MAX(0x118, 0xf)
+  MXL_DPP_MAX(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
+  MXL_DPP_MAX(0x143, 0xc)  // row_bcast:31 into rows 2 and 3
+#undef MXL_DPP_MAX
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);
+  return v;
+}
+
+// Route token t with the calling wavefront: ids / weights [t * topk + r] for r < topk;
+// returns the lane's id (lane r < topk holds selection r, other lanes -1).
+template <bool BF16, int NS>
+__device__ __forceinline__ int32_t route_token(const void* __restrict__ logits, int64_t t, int E, int topk,
+                                               bool renorm, int lane, int32_t* __restrict__ ids,
+                                               float* __restrict__ weights) {
+  uint32_t key[NS];   // of the logits not yet taken, else 0
+  uint64_t left[NS];  // the lanes whose logit is not yet taken
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const int i = lane + 64 * j;
+    float x = 0.0f;
+    if (i < E) x = BF16 ? bf16_to_f32(static_cast<const uint16_t*>(logits)[t * E + i])
+                        : static_cast<const float*>(logits)[t * E + i];
+    key[j] = i < E ? order_key(x) : 0u;
+    left[j] = __ballot(i < E);
+  }
+  float my_x = 0.0f;
+  int32_t my_id = -1;
+  float top = 0.0f, part = 0.0f;
+  for (int r = 0; r < topk; ++r) {
+    uint32_t best = key[0];
+#pragma unroll
+    for (int j = 1; j < NS; ++j) best = key[j] > best ? key[j] : best;
+    best = wave_max_u32(best);
+    const float x = key_value(best);
+    if (r == 0) {
+      top = x;
+      if (!renorm) {
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+          if (lane + 64 * j < E) part = part + mx_exp(key_value(key[j]) - top);
+      }
+    }
+    int idx = 0;  // the lowest expert left with that key
+#pragma unroll
+    for (int j = NS - 1; j >= 0; --j) {
+      const uint64_t m = __ballot(key[j] == best) & left[j];
+      if (m) idx = 64 * j + __builtin_ctzll(m);
+    }
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+      if (j == idx >> 6) {
+        left[j] &= ~(1ull << (idx & 63));
+        if (lane == (idx & 63)) key[j] = 0u;
+      }
+    if (lane == r) {
+      my_x = x;
+      my_id = idx;
+    }
+  }
+  const float e = lane < topk ? mx_exp(my_x - top) : 0.0f;
+  const float denom = wave_sum(renorm ? e : part);
+  if (lane < topk) {
+    ids[t * topk + lane] = my_id;
+    weights[t * topk + lane] = e / denom;
+  }
+  return my_id;
+}
+
+// Up to kRouterSingleTokens tokens, T * topk <= 1024 routes: routing and the token sort in one
+// workgroup, a token per wavefront (256 experts, top 8: 1 / 16 tokens 6.3 / 7.8 us;
+// 17 / 64 tokens 8.9 / 18.0, with router_kernel ahead of the sort 7.7 / 8.1).
+constexpr int kRouterSingleTokens = 16;
+template <bool BF16, int NS>
+__global__ __launch_bounds__(kChunk) void router_single_kernel(const void* __restrict__ logits, int64_t T, int E,
+                                                              int topk, int renorm, int32_t* __restrict__ ids,
+                                                              float* __restrict__ weights,
+                                                              int64_t* __restrict__ expert_offsets,
+                                                              int32_t* __restrict__ sorted_routes,
+                                                              int32_t* __restrict__ inverse) {
+  __shared__ int32_t whist[(kChunk / 64) * kSingleMaxExperts];
+  __shared__ int32_t tot[2][kSingleMaxExperts];
+  __shared__ int32_t sids[kChunk];
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  for (int64_t tok = w; tok < T; tok += kChunk / 64) {
+    const int32_t id = route_token<BF16, NS>(logits, tok, E, topk, renorm != 0, lane, ids, weights);
+    if (lane < topk) sids[tok * topk + lane] = id;
+  }
+  __syncthreads();
+  const int64_t R = T * topk;
+  single_chunk_sort(t < R ? sids[t] : -1, R, E, expert_offsets, sorted_routes, inverse, whist, tot);
+}
+
+// Routing only: ids and weights, sorted by mxl_moe_route afterwards.
+template <bool BF16, int NS>
 __global__ __launch_bounds__(256) void router_kernel(const void* __restrict__ logits, int64_t T, int E, int topk,
                                                      int renorm, int32_t* __restrict__ ids,
                                                      float* __restrict__ weights) {
   const int64_t tok = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tok < T) route_token<BF16>(logits, tok, E, topk, renorm != 0, threadIdx.x & 63, ids, weights);
+  if (tok < T) route_token<BF16, NS>(logits, tok, E, topk, renorm != 0, threadIdx.x & 63, ids, weights);
 }
 
 // One thread: 8 consecutive hidden columns of one token.
@@ -520,6 +523,12 @@ extern "C" int mxl_moe_route(const int32_t* topk_ids, int64_t T, int64_t topk, i
     MXL_CHECK_LAUNCH("mxl_moe_route(single)");
     return MXL_OK;
   }
+  if (C > 1 && C <= kSortMaxChunks && E <= kSingleMaxExperts) {
+    route_sort_kernel<<<dim3((unsigned)C), kChunk, (kChunk / 64 + 4) * E * sizeof(int32_t), s>>>(
+        topk_ids, R, (int)C, (int)E, expert_offsets, sorted_routes, inverse);
+    MXL_CHECK_LAUNCH("mxl_moe_route(sort)");
+    return MXL_OK;
+  }
   int32_t* counts = (int32_t*)workspace;
   if (C > 0 && C * E <= kCountScanMaxEntries && E <= 1024) {
     route_count_scan_kernel<<<1, kChunk, (C * E + 2 * E) * sizeof(int32_t), s>>>(topk_ids, R, C, (int)E, counts,
@@ -541,10 +550,27 @@ extern "C" int mxl_moe_route(const int32_t* topk_ids, int64_t T, int64_t topk, i
   return MXL_OK;
 }
 
-// Router workspace: the chunk histograms of the two-launch schedule, or, for shapes the
-// fused schedules do not take, mxl_moe_route's.
+// Router workspace: mxl_moe_route's.
 extern "C" int64_t mxl_moe_router_workspace_bytes(int64_t T, int64_t topk, int64_t E) {
   return mxl_moe_route_workspace_bytes(T, topk, E);
+}
+
+// The routing launch: routing alone, or (expert_offsets set) with the sort.
+template <bool BF16, int NS>
+static void launch_router(const void* logits, int64_t T, int64_t E, int64_t topk, int renorm, float* weights,
+                          int32_t* ids, int32_t* sorted_routes, int64_t* expert_offsets, int32_t* inverse,
+                          hipStream_t s) {
+  if (expert_offsets)
+    router_single_kernel<BF16, NS><<<1, kChunk, 0, s>>>(logits, T, (int)E, (int)topk, renorm, ids, weights,
+                                                        expert_offsets, sorted_routes, inverse);
+  else
+    router_kernel<BF16, NS><<<(unsigned)((T + 3) / 4), 256, 0, s>>>(logits, T, (int)E, (int)topk, renorm, ids,
+                                                                    weights);
+}
+template <bool BF16, class... Args>
+static void launch_router_slots(int64_t E, const void* logits, int64_t T, Args... args) {
+  if (E <= 256) launch_router<BF16, 4>(logits, T, E, args...);
+  else launch_router<BF16, kRouterSlots>(logits, T, E, args...);
 }
 
 extern "C" int mxl_moe_router(const void* logits, int logits_bf16, int64_t T, int64_t E, int64_t topk,
@@ -562,37 +588,15 @@ extern "C" int mxl_moe_router(const void* logits, int logits_bf16, int64_t T, in
                 (long long)mxl_moe_router_workspace_bytes(T, topk, E));
   hipStream_t s = (hipStream_t)stream;
   const int renorm = renormalize ? 1 : 0;
-  if (R <= kChunk) {  // routing and the sort in one workgroup (also T = 0: the offsets)
-    if (logits_bf16)
-      router_single_kernel<true><<<1, kChunk, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids, topk_weights,
-                                                      expert_offsets, sorted_routes, inverse);
-    else
-      router_single_kernel<false><<<1, kChunk, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids, topk_weights,
-                                                       expert_offsets, sorted_routes, inverse);
-    MXL_CHECK_LAUNCH("mxl_moe_router(single)");
-    return MXL_OK;
-  }
-  int32_t* counts = (int32_t*)workspace;
-  if (kChunk % topk == 0 && C * E <= kCountScanMaxEntries) {
-    // chunks of whole tokens: routing with the chunk histograms, then the scan and scatter
-    if (logits_bf16)
-      router_hist_kernel<true><<<dim3((unsigned)C), kChunk, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids,
-                                                                    topk_weights, counts);
-    else
-      router_hist_kernel<false><<<dim3((unsigned)C), kChunk, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids,
-                                                                     topk_weights, counts);
-    MXL_CHECK_LAUNCH("mxl_moe_router(hist)");
-    route_scan_scatter_kernel<<<dim3((unsigned)C), kChunk, 0, s>>>(topk_ids, R, C, (int)E, counts, expert_offsets,
-                                                                   sorted_routes, inverse);
-    MXL_CHECK_LAUNCH("mxl_moe_router(scatter)");
-    return MXL_OK;
-  }
-  const unsigned blocks = (unsigned)((T + 3) / 4);
+  // few tokens (also T = 0: the offsets): routing and the sort in one launch
+  const bool single = R <= kChunk && T <= kRouterSingleTokens;
+  int64_t* const offsets = single ? expert_offsets : nullptr;
   if (logits_bf16)
-    router_kernel<true><<<blocks, 256, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids, topk_weights);
+    launch_router_slots<true>(E, logits, T, topk, renorm, topk_weights, topk_ids, sorted_routes, offsets, inverse, s);
   else
-    router_kernel<false><<<blocks, 256, 0, s>>>(logits, T, (int)E, (int)topk, renorm, topk_ids, topk_weights);
+    launch_router_slots<false>(E, logits, T, topk, renorm, topk_weights, topk_ids, sorted_routes, offsets, inverse, s);
   MXL_CHECK_LAUNCH("mxl_moe_router(route)");
+  if (single) return MXL_OK;
   return mxl_moe_route(topk_ids, T, topk, E, sorted_routes, expert_offsets, inverse, workspace, workspace_bytes,
                        stream);
 }

@@ -775,7 +775,7 @@ def moe_router(router_logits: torch.Tensor, top_k: int, renormalize: bool = True
     """Router logits [T, E] (fp32 or bf16) -> (topk_weights f32 [T, k], topk_ids i32 [T, k],
     sorted_routes i32 [T k], expert_offsets i64 [E+1], inverse i32 [T k]): softmax, top-k
     (ties to the lower expert), renormalization and the stable token sort of ``moe_route``,
-    in one launch up to 1024 routes (vLLM's fused top-k softmax + the routing of
+    in one launch up to 16 tokens (vLLM's fused top-k softmax + the routing of
     ``route_mxfp8_out``, as qwen35_router_quant_out fuses them, src/vllm_mach/mxfp6/moe.py:142-152).
     """
     _check_cuda(router_logits)
