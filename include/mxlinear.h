@@ -439,9 +439,8 @@ int mxl_moe_route(const int32_t* topk_ids, int64_t T, int64_t topk, int64_t E, i
  * topk_weights fp32 [T, topk] = exp(x - max) / sum, the sum over the selected experts
  * (renormalize = 1) or over all experts (0), with this library's binary32 exp.  Then
  * sorted_routes / expert_offsets / inverse exactly as mxl_moe_route writes them for
- * those ids.  One launch while T * topk <= 1024; two while topk divides 1024 and the
- * chunk histograms fit one workgroup; otherwise the routing and mxl_moe_route's
- * launches.  Replaces vLLM's fused top-k softmax (select_experts: softmax, topk,
+ * those ids.  One launch up to 16 tokens (T * topk <= 1024); otherwise the routing and
+ * mxl_moe_route's launches.  Replaces vLLM's fused top-k softmax (select_experts: softmax, topk,
  * renormalize) and the routing of route_mxfp8_out, fused as the reference's
  * qwen35_router_quant_out fuses them (src/vllm_mach/mxfp6/moe.py:142-152). */
 int64_t mxl_moe_router_workspace_bytes(int64_t T, int64_t topk, int64_t E);

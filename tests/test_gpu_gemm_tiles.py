@@ -156,3 +156,27 @@ def test_noalloc_takes_a_plan_past_its_scratch(pkg, oracle_mod, dev):
               out.data_ptr(), N, torch.cuda.current_stream(dev).cuda_stream)
     ref = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, None)
     _check(out.float().cpu().numpy(), ref.float().cpu().numpy())
+
+
+@pytest.mark.parametrize("N,K,fmt,gathered", [(200, 128, 2, False), (384, 1152, 3, True), (264, 2048, 0, True)])
+def test_grouped_tiles(pkg, dev, monkeypatch, N, K, fmt, gathered):
+    """Experts without rows, of one row, and either side of a 64- and a 128-row block, against the
+    per-expert kernel; ragged N, one slice and an odd count of them."""
+    ops = pkg.ops
+    counts = [0, 1, 64, 65, 0, 128, 129, 200, 63, 3]
+    E, R = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(N + K)
+    width = K if fmt == 0 else K * 3 // 4
+    codes = torch.randint(0, 0x70 if fmt == 0 else 256, (E, N, width), generator=g, dtype=torch.uint8).to(dev)
+    scales = torch.randint(118, 122, (E, N, K // 32), generator=g, dtype=torch.uint8).to(dev)
+    w, sw = ops.pack_weight(codes.view(torch.float8_e4m3fn) if fmt == 0 else codes, scales, fmt)
+    offsets = torch.tensor([0] + counts).cumsum(0).to(dev)
+    index = torch.randperm(R, generator=g).to(torch.int32).to(dev) if gathered else None
+    a, sa = torch.ops.mach_amd.quantize_mxfp8(_act((R + 1) // 2 if gathered else R, K, 4).to(dev), 0)
+    args = (a, sa, index, 2 if gathered else 1, offsets, R, w, sw, N, K, fmt)
+    got = []
+    for fields in (dict(kernel=ops.KERNEL_WIDE), dict(kernel=ops.KERNEL_WIDE, tile_m=4), dict(kernel=ops.KERNEL_GENERIC)):
+        monkeypatch.setattr(ops, "_tuning", _options(ops, **fields))
+        got.append(torch.ops.mach_amd.grouped_gemm(*args).float().cpu().numpy())
+    assert (got[0] == got[1]).all()  # whole-K sums are the same chain of MFMAs
+    _check(got[0], got[2])

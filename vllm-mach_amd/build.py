@@ -37,6 +37,7 @@ FLAGS = [
 FILE_FLAGS: dict[str, list[str]] = {
     # the block-FP8 tiles fold each MFMA's result with vector instructions
     "gemm_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "gemm_tile_grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "gemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     # the dense MX wide launches: the iterative ILP schedule
     "gemm_wide_mx.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],

@@ -1276,7 +1276,7 @@ static GroupedPlan plan_grouped(int64_t a_rows, int64_t num_experts, int64_t rou
     else if (routed_rows <= 96 * num_experts && K <= kTileK) stream_mt = kGroupedStreamWideMT;
   }
   if (stream_mt && !stream_grouped_eligible(K, num_experts, w_fmt, stream_mt)) stream_mt = 0;
-  const bool wide_ok = K % 256 == 0 && a_rows * K < (int64_t(1) << 32) && num_experts <= kWideGroupedMaxExperts;
+  const bool wide_ok = a_rows * K < (int64_t(1) << 32) && num_experts <= kWideGroupedMaxExperts;
   if (!stream_mt && force != kGeneric && wide_ok && (force == kWide || routed_rows >= 32 * num_experts))
     return GroupedPlan{kWide, 0, o.tile_m == 4 ? 4 : 8};
   if (stream_mt) return GroupedPlan{kStream, stream_mt, 0};
@@ -1321,7 +1321,7 @@ static int grouped_common(const void* a, const void* sa, int64_t a_rows, const i
   MXL_CHECK_ARG(default_epilogue(o), "mxl_grouped_gemm: bf16 output without scaling only");
   const GroupedPlan gp = plan_grouped(a_rows, num_experts, routed_rows, K, w_fmt, o);
   const int stream_mt = gp.stream_mt;
-  if (gp.kernel == kWide) {
+  if (gp.kernel == kWide && wide_tiles_eligible(a_rows, N, K, false)) {
     // enough rows per expert on average for 128-row blocks: the wide kernel
     GemmParams p{};
     p.a = (const uint8_t*)a; p.sa = sa; p.w = (const uint8_t*)w_tiled; p.sw = sw_tiled;

@@ -43,14 +43,15 @@ __device__ __forceinline__ I wide_logical(I L, I G) {
 }
 
 // Workgroups per CU the kernel is compiled for: the 2 x 2-wave tiles by their size (LDS and
-// registers), the grouped four-wave tiles two, the dense ones one.
+// registers), the grouped tiles two, the dense four-wave tiles one.
 template <int MT, int NT, bool GROUPED, int WM>
 struct WidePerCu {
   static constexpr int value = WM == 2 ? (MT * NT > 16 ? 1 : MT * NT > 8 ? 2 : 3) : GROUPED ? 2 : 1;
 };
 
 // Arrangement of the four waves: WM = 1 side by side (each all MT m-tiles by NT n-tiles;
-// gemm_wide.hip), WM = 2 two by two (each MT / 2 m-tiles by 2 NT n-tiles; gemm_tile.hip).
+// gemm_wide.hip), WM = 2 two by two (each MT / 2 m-tiles by 2 NT n-tiles; gemm_tile.hip).  Grouped
+// launches (WM = 1 by name) are two by two as well (gemm_tile_grouped.hip).
 template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED, int WM>
 struct WideKernel;
 
@@ -63,5 +64,9 @@ __global__ __launch_bounds__(256, (WidePerCu<MT, NT, GROUPED, WM>::value)) void 
 // The dense 2 x 2-wave launch of `grid` workgroups.
 hipError_t launch_wide_tiles(int fmt, bool block, const WideConfig& c, const GemmParams& p, const WideGrid& g,
                              int64_t grid, hipStream_t s);
+
+// The grouped (MoE) launch of `grid` persistent workgroups (gemm_tile_grouped.hip).
+hipError_t launch_wide_grouped(int fmt, const WideConfig& c, const GemmParams& p, const WideGrid& g, int64_t grid,
+                               hipStream_t s);
 
 }  // namespace mxl

@@ -1,5 +1,5 @@
-// Wide-tile, LDS-pipelined GEMM for prefill-sized M on gfx950 (MX, block-FP8,
-// dense and MoE-grouped): the four-wave tiles, the planner of the dense 2 x 2-wave tiles
+// Wide-tile, LDS-pipelined GEMM for prefill-sized M on gfx950 (MX and block-FP8,
+// dense): the four-wave tiles, the planner of the dense 2 x 2-wave tiles
 // (gemm_tile.hip; what the automatic dense plans run) and the split reduce of both.
 //
 // Workgroup tile: 128 rows x 64*NT columns (NT = 1, 2 or 4), four wavefronts.
@@ -10,8 +10,7 @@
 // of a wave writes 4 or 16 bytes at LDS base + 4i / 16i, no staging
 // registers) into a ring of K128 stage slots (four, or three for NT = 4 whose
 // 53 KiB stages would not fit four times), issued two or three stages ahead of
-// the MFMAs; the grouped variant runs two workgroups per CU with two slots each,
-// one stage ahead.  A slot holds
+// the MFMAs.  A slot holds
 //   A    8 m-tiles x 2 KiB: chunk (m-tile i, half h) holds rows 16 i + 8 h ..
 //        + 7 whole (the slice's 128 bytes per row), the eight 16-byte pieces of
 //        row r permuted by piece ^ a_swz(r).  The copy is row-major because the
@@ -42,9 +41,7 @@
 // tile, and a second kernel sums them in split order and writes the rows.  When the whole-K tiles
 // leave a partial last round (more tiles than CUs), the same launch runs the
 // leftover tiles split in K: workgroup L computes whole-K tile L and then unit L
-// of the split leftovers, so no CU waits for a second launch.  The grouped variant
-// walks experts' row ranges (expert_offsets) on device, so the launch needs no
-// host-side counts.
+// of the split leftovers, so no CU waits for a second launch.
 #include "gemm_wide.h"
 
 // the copies set M0 (the LDS base of a global->LDS load) themselves
@@ -76,9 +73,6 @@ struct WideSlot {
   static constexpr int SBC = BLOCK ? 0 : NT;
   static constexpr int COPIES = ACH + 2 * NT + SBC;
 };
-
-// Ring slots of the grouped variant, which runs two workgroups per CU.
-constexpr int kWideGroupedSlots = 2;
 
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
@@ -298,10 +292,9 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 
 }  // namespace
 
-// One output tile: rows [row_base, hi) of m-block rows (hi bounds the valid rows
-// of a grouped expert), n-block nb, K split `split`; w / sw are the expert's
-// weights.  The ring and the scale ring are the workgroup's LDS.
-template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED>
+// One output tile: rows [row_base, hi) of m-block rows, n-block nb, K split `split`.  The ring and
+// the scale ring are the workgroup's LDS.
+template <int FMT, int MT, int NT, bool BLOCK>
 __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int64_t row_base, int64_t hi,
                                           const uint8_t* w, const uint8_t* sw, int64_t nb, int64_t split,
                                           float* pdst, uint8_t* ring, uint8_t* sa_ring, float* sb_stage,
@@ -311,7 +304,7 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
   constexpr int BM = 16 * MT;
   auto a_row = [&](int64_t row) -> int64_t {
     if (row >= hi) row = hi - 1;  // padding rows copy a valid row; their outputs are not stored
-    return (GROUPED && p.row_index) ? (int64_t)(p.row_index[row] / p.row_div) : row;
+    return row;
   };
   const int64_t ntiles_total = (p.N + 15) / 16;
   const int64_t nt_wave = (nb * 4 + wv) * NT;
@@ -376,42 +369,7 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
       else copy4(static_cast<const uint8_t*>(p.sa) + (tb >> 2) * 4 * p.sa_ss, L.sa_piece[j], dst);
     }
   }
-  if constexpr (GROUPED) {
-    // Two workgroups per CU, each with a two-slot ring and one register set: step tt
-    // waits for its own copies of stage tt (issued in the step before, the last ones
-    // in flight), a barrier hands stage tt to every wave and frees the slot read in
-    // the step before, stage tt + 1 is copied into it, then stage tt is read and
-    // multiplied.  The other workgroup's steps run while this one waits on LDS
-    // reads, copies or its prologue and epilogue.
-    constexpr int R = kWideGroupedSlots;
-    static_assert(4 % R == 0, "the four steps below rotate the slots");
-    if (tb < te) wide_copy<FMT, MT, NT, BLOCK>(p, ring, tb, wv, lane, L, sa_ring);
-    WideRegs<MT, NT, BLOCK> x;
-#define MXL_WIDE_STEP2(I_)                                                                              \
-  {                                                                                                   \
-    const int64_t tt = t0 + I_;                                                                       \
-    if (tt < te) {                                                                                    \
-      wait_vm<0>();                                                                                   \
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                            \
-      wide_barrier();                                                                                 \
-      if (tt + 1 < te)                                                                                \
-        wide_copy<FMT, MT, NT, BLOCK>(p, ring + ((I_ + 1) % R) * S::BYTES, tt + 1, wv, lane, L, sa_ring); \
-      wide_read<FMT, MT, NT, BLOCK>(ring + (I_ % R) * S::BYTES, sa_ring + ((tt >> 2) % 3) * S::RING_ENTRY, \
-                                        (int)(tt & 3), wv, lane, q, r, x);                           \
-      if (BLOCK) x.sbv = sb_stage[tt - tb];                                                           \
-      wide_mfma<FMT, MT, NT, BLOCK>(x, acc);                                                         \
-    }                                                                                                 \
-  }
-    // four steps per iteration: tb is a multiple of 4, so each step's slice index
-    // (tt & 3) is a compile-time value and the per-slice lane offsets stay in registers
-    for (int64_t t0 = tb; t0 < te; t0 += 4) {
-      MXL_WIDE_STEP2(0)
-      MXL_WIDE_STEP2(1)
-      MXL_WIDE_STEP2(2)
-      MXL_WIDE_STEP2(3)
-    }
-#undef MXL_WIDE_STEP2
-  } else if (tb < te) {
+  if (tb < te) {
     constexpr int R = S::SLOTS;
     // prologue: stages tb .. tb + R - 1 fill the ring; stage tb is read into registers
 #pragma unroll
@@ -478,7 +436,7 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
   // stores straight from the accumulator layout would cost a store instruction
   // per 64 values with 64-bit address arithmetic for each.
   constexpr int TW = 64 * NT, ST = TW + 4;
-  static_assert(BM * ST * 4 <= (GROUPED ? kWideGroupedSlots : S::SLOTS) * S::BYTES, "epilogue tile exceeds the ring");
+  static_assert(BM * ST * 4 <= S::SLOTS * S::BYTES, "epilogue tile exceeds the ring");
   if (pdst) {
     // fp32 split partials go straight from the accumulators, in MFMA fragment order: the
     // tile's block at pdst holds fragment f = m-tile * 4 NT + n-tile as 64 lanes x 4
@@ -577,19 +535,14 @@ __device__ __forceinline__ void wide_tile(const GemmParams& p, int64_t kps, int6
   }
 }
 
-// Largest number of experts the grouped variant keeps in LDS.
-constexpr int kWideMaxExperts = (int)kWideGroupedMaxExperts;
-
-// The grouped variant runs two workgroups per CU (at most 256 registers per lane and
-// half the LDS each).
-template <int FMT, int MT, int NT, bool BLOCK, bool GROUPED>
-struct WideKernel<FMT, MT, NT, BLOCK, GROUPED, 1> {
+template <int FMT, int MT, int NT, bool BLOCK>
+struct WideKernel<FMT, MT, NT, BLOCK, false, 1> {
 static __device__ __forceinline__ void run(const GemmParams& p, const WideGrid& g) {
   using S = WideSlot<MT, NT, BLOCK>;
   constexpr int BM = 16 * MT;
-  // the stage ring (dense: the LDS budget of one workgroup per CU; grouped: two slots);
-  // after the last stage it holds the output tile of the epilogue
-  __shared__ __attribute__((aligned(16))) uint8_t ring[(GROUPED ? kWideGroupedSlots : S::SLOTS) * S::BYTES];
+  // the stage ring (the LDS budget of one workgroup per CU); after the last stage it holds
+  // the output tile of the epilogue
+  __shared__ __attribute__((aligned(16))) uint8_t ring[S::SLOTS * S::BYTES];
   __shared__ __attribute__((aligned(16))) uint8_t sa_ring[S::SA_RING ? 3 * S::RING_ENTRY : 16];
   // block-FP8: each wave's weight block scales of the tile's K range
   __shared__ float sb_lds[BLOCK ? 4 * kWideBlockStages : 1];
@@ -597,106 +550,37 @@ static __device__ __forceinline__ void run(const GemmParams& p, const WideGrid& 
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r = lane & 15, q = lane >> 4;
 
-  if (!GROUPED) {
-    // XCD-aware remap of the linear workgroup id: the m-blocks sharing a weight
-    // slice run consecutively on one XCD
-    const int64_t logical = wide_logical(blockIdx.x, gridDim.x);
-    constexpr int TW = 64 * NT;
-    float* const sbw = sb_lds + (BLOCK ? wv * kWideBlockStages : 0);
-    const uint8_t* const sw = static_cast<const uint8_t*>(p.sw);
-    if (g.rem_tiles == 0) {
-      const int64_t local = logical % g.tiles, split = logical / g.tiles;
-      int64_t mb, nb;
-      wide_coords(local, g.mblocks, g.nblocks, g.group_m, mb, nb);
-      // split partials: the tile's fragment-ordered block, [split][tile][BM x TW]
-      float* const pdst = p.S == 1 ? nullptr : p.partial + (split * g.tiles + local) * BM * TW;
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, split, pdst, ring,
-                                                 sa_ring, sbw, t, lane, wv, r, q);
-      return;
-    }
-    // one-launch hybrid: the whole-K tile, then the remainder unit (if any)
-    if (logical < g.tiles) {
-      int64_t mb, nb;
-      wide_coords(logical, g.mblocks, g.nblocks, g.group_m, mb, nb);
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, 0, nullptr, ring,
-                                                 sa_ring, sbw, t, lane, wv, r, q);
-    }
-    if (logical < g.rem_tiles * g.S2) {
-      const int64_t local = logical % g.rem_tiles, split = logical / g.rem_tiles;
-      int64_t mb, nb;
-      wide_coords(g.rem_tile0 + local, g.mblocks, g.nblocks, g.group_m, mb, nb);
-      __syncthreads();  // the first tile's epilogue reads of the ring are done
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt2, mb * BM, p.M, p.w, sw, nb, split,
-                                                 p.partial + (split * g.rem_tiles + local) * BM * TW, ring, sa_ring,
-                                                 sbw, t, lane, wv, r, q);
-    }
+  // XCD-aware remap of the linear workgroup id: the m-blocks sharing a weight
+  // slice run consecutively on one XCD
+  const int64_t logical = wide_logical(blockIdx.x, gridDim.x);
+  constexpr int TW = 64 * NT;
+  float* const sbw = sb_lds + (BLOCK ? wv * kWideBlockStages : 0);
+  const uint8_t* const sw = static_cast<const uint8_t*>(p.sw);
+  if (g.rem_tiles == 0) {
+    const int64_t local = logical % g.tiles, split = logical / g.tiles;
+    int64_t mb, nb;
+    wide_coords(local, g.mblocks, g.nblocks, g.group_m, mb, nb);
+    // split partials: the tile's fragment-ordered block, [split][tile][BM x TW]
+    float* const pdst = p.S == 1 ? nullptr : p.partial + (split * g.tiles + local) * BM * TW;
+    wide_tile<FMT, MT, NT, BLOCK>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, split, pdst, ring,
+                                               sa_ring, sbw, t, lane, wv, r, q);
     return;
   }
-
-  // Grouped: persistent workgroups.  The experts' BM-row block counts are
-  // prefix-summed once per workgroup into LDS; each workgroup then walks the
-  // tiles L = blockIdx, blockIdx + grid, ... of the routed (m-block x n-block)
-  // grid, n-blocks fastest (the same XCD remap, so a workgroup stays on its XCD's
-  // tiles), and finds its expert by a parallel search of the prefix.  Only the prefix
-  // stays in LDS (two workgroups share a CU's LDS); a tile reads its expert's row range
-  // from expert_offsets.
-  __shared__ int32_t sh_pre[kWideMaxExperts + 1];   // m-blocks before expert e
-  __shared__ int32_t sh_hit;
-  const int E = (int)g.num_experts;
-  // block counts per thread chunk, then a block-wide inclusive scan of the chunk sums
-  // (in the ring, which holds no stage yet)
-  const int chunk = (E + 255) / 256;
-  const int e0 = t * chunk < E ? t * chunk : E, e1 = e0 + chunk < E ? e0 + chunk : E;
-  int cnt = 0;
-  for (int e = e0; e < e1; ++e)
-    cnt += (int)((p.expert_offsets[e + 1] - p.expert_offsets[e] + BM - 1) / BM);
-  int32_t* const sh_scan = reinterpret_cast<int32_t*>(ring);
-  sh_scan[t] = cnt;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int v = t >= off ? sh_scan[t - off] : 0;
-    __syncthreads();
-    sh_scan[t] += v;
-    __syncthreads();
+  // one-launch hybrid: the whole-K tile, then the remainder unit (if any)
+  if (logical < g.tiles) {
+    int64_t mb, nb;
+    wide_coords(logical, g.mblocks, g.nblocks, g.group_m, mb, nb);
+    wide_tile<FMT, MT, NT, BLOCK>(p, g.kt_per_split, mb * BM, p.M, p.w, sw, nb, 0, nullptr, ring,
+                                               sa_ring, sbw, t, lane, wv, r, q);
   }
-  int base = sh_scan[t] - cnt;  // exclusive prefix of this thread's chunk
-  for (int e = e0; e < e1; ++e) {
-    sh_pre[e] = base;
-    base += (int)((p.expert_offsets[e + 1] - p.expert_offsets[e] + BM - 1) / BM);
-  }
-  if (t == 255) sh_pre[E] = sh_scan[255];
-  __syncthreads();
-  const int64_t total_mb = sh_pre[E];
-  // the routed tiles only (the launch's m-block count is a bound): the XCD remap then
-  // spreads them evenly, whatever the tile order
-  const int64_t Gt = (total_mb < g.mblocks ? total_mb : g.mblocks) * g.nblocks;
-  const int64_t per = Gt >> 3, extra = Gt & 7;
-  for (int64_t Lid = blockIdx.x; Lid < Gt; Lid += gridDim.x) {
-    const int64_t xcd = Lid & 7;
-    const int64_t logical = xcd * per + (xcd < extra ? xcd : extra) + (Lid >> 3);
-    // n-blocks fastest: an expert block's n-blocks are consecutive, so they run on one
-    // XCD and its gathered activation rows are fetched into that L2 once
-    const int64_t nb = logical % g.nblocks;
-    const int64_t mb = logical / g.nblocks;
-    if (mb >= total_mb) continue;  // beyond the routed m-blocks (uniform)
-    if (t == 0) sh_hit = 0;
-    __syncthreads();
-    for (int e = t; e < E; e += 256)
-      if (sh_pre[e] <= mb && mb < sh_pre[e + 1]) sh_hit = e;
-    __syncthreads();
-    const int e = __builtin_amdgcn_readfirstlane(sh_hit);
-    const int64_t rb = p.expert_offsets[e] + (mb - sh_pre[e]) * BM, rhi = p.expert_offsets[e + 1];
-    const uint8_t* we = p.w + e * p.w_expert_stride;
-    const uint8_t* swe = static_cast<const uint8_t*>(p.sw) + e * p.sw_expert_stride;
-    // a 128-row block with at most 64 routed rows (an expert's last block) runs the
-    // 64-row tile path in the same ring: half the activation copies and MFMAs
-    if (MT == 8 && __builtin_amdgcn_readfirstlane((int)(rhi - rb)) <= 64)
-      wide_tile<FMT, (MT == 8 ? 4 : MT), NT, BLOCK, GROUPED>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr,
-                                                             ring, sa_ring, sb_lds, t, lane, wv, r, q);
-    else
-      wide_tile<FMT, MT, NT, BLOCK, GROUPED>(p, g.kt_per_split, rb, rhi, we, swe, nb, 0, nullptr, ring, sa_ring,
-                                             sb_lds, t, lane, wv, r, q);
-    __syncthreads();  // the epilogue's LDS reads are done before the next tile's copies
+  if (logical < g.rem_tiles * g.S2) {
+    const int64_t local = logical % g.rem_tiles, split = logical / g.rem_tiles;
+    int64_t mb, nb;
+    wide_coords(g.rem_tile0 + local, g.mblocks, g.nblocks, g.group_m, mb, nb);
+    __syncthreads();  // the first tile's epilogue reads of the ring are done
+    wide_tile<FMT, MT, NT, BLOCK>(p, g.kt2, mb * BM, p.M, p.w, sw, nb, split,
+                                               p.partial + (split * g.rem_tiles + local) * BM * TW, ring, sa_ring,
+                                               sbw, t, lane, wv, r, q);
   }
 }
 };
@@ -972,42 +856,41 @@ bool wide_gemm_eligible(int64_t M, int64_t K) { return M >= 64 && K % 256 == 0 &
 
 #endif  // MXL_WIDE_MX_DENSE_ONLY
 
-template <int FMT, int MT, bool BLOCK, bool GROUPED>
+template <int FMT, int MT, bool BLOCK>
 static hipError_t launch_wide_mt(const WideConfig& c, const GemmParams& p, const WideGrid& g, int64_t grid,
                                  hipStream_t s) {
   const dim3 gr((unsigned)grid), blk(256);
   if (c.NT == 4) {
-    if constexpr (GROUPED) return hipErrorInvalidValue;  // the grouped variant runs NT <= 2 (LDS)
-    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 4, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
+    hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 4, BLOCK, false, 1>), gr, blk, 0, s, p, g);
   } else if (c.NT == 2) {
-    hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 2, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
+    hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 2, BLOCK, false, 1>), gr, blk, 0, s, p, g);
   } else if (c.NT == 1) {
     if constexpr (MT == 4) return hipErrorInvalidValue;  // 64 x 64 tiles are not instantiated
-    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 1, BLOCK, GROUPED, 1>), gr, blk, 0, s, p, g);
+    else hipLaunchKernelGGL((gemm_wide_kernel<FMT, MT, 1, BLOCK, false, 1>), gr, blk, 0, s, p, g);
   } else {
     return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-template <int FMT, bool BLOCK, bool GROUPED>
+template <int FMT, bool BLOCK>
 static hipError_t launch_wide_fmt(const WideConfig& c, const GemmParams& p, const WideGrid& g, int64_t grid,
                                   hipStream_t s) {
-  if (c.MT == 8) return launch_wide_mt<FMT, 8, BLOCK, GROUPED>(c, p, g, grid, s);
-  if (c.MT == 4) return launch_wide_mt<FMT, 4, BLOCK, GROUPED>(c, p, g, grid, s);
+  if (c.MT == 8) return launch_wide_mt<FMT, 8, BLOCK>(c, p, g, grid, s);
+  if (c.MT == 4) return launch_wide_mt<FMT, 4, BLOCK>(c, p, g, grid, s);
   return hipErrorInvalidValue;
 }
 
-// The dense MX launches (gemm_wide_mx.hip compiles this file again with
-// MXL_WIDE_MX_DENSE_ONLY for them alone, under its own scheduling flags; the block-FP8
-// and grouped launches stay in this translation unit).
+// The MX launches (gemm_wide_mx.hip compiles this file again with MXL_WIDE_MX_DENSE_ONLY
+// for them alone, under its own scheduling flags; the block-FP8 launches stay in this
+// translation unit).
 hipError_t launch_wide_mx_dense(int fmt, const WideConfig& c, const GemmParams& q, const WideGrid& gg, int64_t n,
                                 hipStream_t s)
 #ifdef MXL_WIDE_MX_DENSE_ONLY
 {
-  if (fmt == kE4M3) return launch_wide_fmt<kE4M3, false, false>(c, q, gg, n, s);
-  if (fmt == kE2M3) return launch_wide_fmt<kE2M3, false, false>(c, q, gg, n, s);
-  if (fmt == kE3M2) return launch_wide_fmt<kE3M2, false, false>(c, q, gg, n, s);
+  if (fmt == kE4M3) return launch_wide_fmt<kE4M3, false>(c, q, gg, n, s);
+  if (fmt == kE2M3) return launch_wide_fmt<kE2M3, false>(c, q, gg, n, s);
+  if (fmt == kE3M2) return launch_wide_fmt<kE3M2, false>(c, q, gg, n, s);
   return hipErrorInvalidValue;
 }
 #else
@@ -1026,10 +909,7 @@ hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const Gemm
     g.mblocks = (p.M + bm - 1) / bm + num_experts;  // bound on the routed m-blocks
     grid = g.mblocks * g.nblocks;
     if (grid > 2 * cu_count()) grid = 2 * cu_count();  // persistent workgroups (two per CU) walk the tiles
-    if (fmt == kE4M3) return launch_wide_fmt<kE4M3, false, true>(c, p, g, grid, s);
-    if (fmt == kE2M3) return launch_wide_fmt<kE2M3, false, true>(c, p, g, grid, s);
-    if (fmt == kE3M2) return launch_wide_fmt<kE3M2, false, true>(c, p, g, grid, s);
-    return hipErrorInvalidValue;
+    return launch_wide_grouped(fmt, c, p, g, grid, s);
   }
   g.mblocks = (p.M + bm - 1) / bm;
   g.tiles = g.mblocks * g.nblocks;
@@ -1039,7 +919,7 @@ hipError_t launch_gemm_wide(int fmt, bool block, const WideConfig& c, const Gemm
   g.group_m = c.WM == 2 && g.mblocks * bm > 1024 ? 1024 / bm : g.mblocks;
   auto dense = [&](const GemmParams& q, const WideGrid& gg, int64_t n) -> hipError_t {
     if (c.WM == 2) return launch_wide_tiles(fmt, block, c, q, gg, n, s);
-    if (block) return fmt == kE4M3 ? launch_wide_fmt<kE4M3, true, false>(c, q, gg, n, s) : hipErrorInvalidValue;
+    if (block) return fmt == kE4M3 ? launch_wide_fmt<kE4M3, true>(c, q, gg, n, s) : hipErrorInvalidValue;
     return launch_wide_mx_dense(fmt, c, q, gg, n, s);
   };
   const int64_t tw = 64 * c.NT;
