@@ -602,7 +602,7 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   if (d.kernel == kWide) {
     const bool auto_tile = o.tile_n == 0 && o.splits == 0 && o.waves == 0 && o.tile_m == 0 && !o.hybrid;
     if (auto_tile && tiles_ok) {
-      d.wide = wide_tiles_config(M, N, K, fmt, block);
+      d.wide = wide_tiles_config(M, N, K, block);
     } else {
       d.wide = wide_config(M, N, K, fmt, o);
       // no 2 x 2-wave block-FP8 tile of 256 columns

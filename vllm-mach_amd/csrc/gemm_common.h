@@ -271,7 +271,7 @@ struct WideConfig {
 WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptions& o = GemmOptions());
 // The 2 x 2-wave tiles (gemm_tile.hip): the shapes they take, and the time model's choice.
 bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block);
-WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool block);
+WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block);
 // Workspace bytes a configuration needs (split partials), 0 when none.
 int64_t wide_workspace_bytes(const WideConfig& c, int64_t M, int64_t N);
 bool wide_gemm_eligible(int64_t M, int64_t K);

@@ -761,8 +761,8 @@ WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptio
 //
 // Time model, fitted to a sweep of every tile and split over 184 dense shapes (M 17..2048, N
 // 256..18432, K 512..17408, MXFP8, MXFP6 and block-FP8 weights rotated out of the caches): a launch
-// costs its fixed time, the stages of the fullest CU, its operands from HBM and its output, which
-// nothing overlaps in the last round.  Its pick runs within 0.9 % of the best of them on average
+// costs its fixed time, the stages of the fullest CU, its output, which nothing overlaps in the last
+// round, and its operands from HBM (at 10.6 TB/s; the same for every choice, so left out below).  Its pick runs within 0.9 % of the best of them on average
 // (the farthest: 722 x 11264 x 896 21.0 us against 18.1, 561 x 1792 x 17408 38.4 against 32.9).
 struct TileCost {
   int MT, NT, resident;   // tile, workgroups per CU
@@ -776,7 +776,7 @@ constexpr TileCost kTileCosts[] = {{16, 4, 1, 4.9, 1.07, 0.402}, {8, 4, 1, 4.3, 
 constexpr double kTileBlockAlone = 1.06, kTileBlockShared = 0.874;
 constexpr double kTileGap = 0.5;                  // a further round's start on a CU, us
 constexpr double kTileReduce = 3.2;               // the split reduce's launch, us
-constexpr double kTileBytesPerUs = 10.6e6, kTileOutBytesPerUs = 2.3e6, kTilePartialBytesPerUs = 6.1e6;
+constexpr double kTileOutBytesPerUs = 2.3e6, kTilePartialBytesPerUs = 6.1e6;
 // the few tiles of a hybrid's remainder: their partials stay in the caches
 constexpr double kTileRemainderBytesPerUs = 8.9e6;
 
@@ -798,10 +798,8 @@ bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
 }
 
 // Tile, split and hybrid of the 2 x 2-wave kernels by the time model.
-WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool block) {
+static WideConfig wide_tiles_choice(int64_t M, int64_t N, int64_t K, bool block) {
   const int64_t KT = (K + kTileK - 1) / kTileK, T = (K + 127) / 128, cus = cu_count();
-  const double weights = (double)N * K * (fmt == kE4M3 ? 1.0 : 0.75) + (double)N * K / 32;
-  const double in = (weights + (double)M * K) / kTileBytesPerUs;
   const double out = 2.0 * M * N / kTileOutBytesPerUs;
   WideConfig best{2, 1, KT};
   double best_us = 1e300;
@@ -824,7 +822,7 @@ WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool bloc
       if ((KT + per - 1) / per != s) continue;
       const int64_t stages = per * 4 < T ? per * 4 : T, n = (tiles * s + cus - 1) / cus;
       const int64_t tail = s == 1 ? wide_tail(t, tiles, cus) : 0;
-      double us = t.fixed + in;
+      double us = t.fixed;
       if (tail) us += work(n - 1, stages) + (4 * tail + cus - 1) / cus * stages * t.quarter + kTileGap;
       else us += work(n, stages);
       if (s == 1) us += out;
@@ -836,12 +834,26 @@ WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, int fmt, bool bloc
     // against 54.1.  (Quarters for the remainder would take 24.3 and 40.3 there.)
     WideConfig h{t.NT, 1, KT};
     if (t.MT == 8 && t.NT == 2 && wide_hybrid(tiles, KT, cus, h) && h.dp_tiles == cus)
-      take(t.fixed + in + work(1, T) + h.kt2 * 4 * t.stage * (block ? kTileBlockShared : 1.0) + kTileReduce +
+      take(t.fixed + work(1, T) + h.kt2 * 4 * t.stage * (block ? kTileBlockShared : 1.0) + kTileReduce +
                (double)(tiles - cus) * 128 * 128 * 8 * h.S2 / kTileRemainderBytesPerUs,
            h);
   }
   best.WM = 2;
   return best;
+}
+
+// The choice is a function of the sizes; a call asks for it up to four times (the workspace query
+// over the formats, then the launch), so each thread keeps its last two (0.6 us each).
+WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
+  struct Last {
+    int64_t M, N, K, cus;
+    WideConfig c;
+  };
+  static thread_local Last last[2] = {};
+  Last& l = last[block];
+  const int64_t cus = cu_count();
+  if (l.M != M || l.N != N || l.K != K || l.cus != cus) l = Last{M, N, K, cus, wide_tiles_choice(M, N, K, block)};
+  return l.c;
 }
 
 int64_t wide_workspace_bytes(const WideConfig& c, int64_t M, int64_t N) {

@@ -149,10 +149,30 @@ class Mxfp8LinearKernel(_Kernel):
         if x.numel() == 0:
             return x.new_empty((*x.shape[:-1], n))
         x2 = _flatten(x, k).contiguous()
-        gemm = ops.mx_gemm_from_float_dual if x2.shape[0] in self.dual_m else ops.mx_gemm_from_float
-        y = gemm(x2, layer.weight, layer.weight_scale, n, layer.mxl_format, self.act_rule)
+        dual = x2.shape[0] in self.dual_m
+        gemm = ops.mx_gemm_from_float_dual if dual else ops.mx_gemm_from_float
+        inner = None if dual else _epilogue_bias(bias, x, n)
+        y = gemm(x2, layer.weight, layer.weight_scale, n, layer.mxl_format, self.act_rule, inner)
         y = y.reshape(*x.shape[:-1], n)
-        return y if bias is None else y + bias
+        return y if bias is inner else y + bias
+
+
+def _epilogue_bias(bias: Optional[torch.Tensor], x: torch.Tensor, n: int) -> Optional[torch.Tensor]:
+    """``bias`` if the GEMM's epilogue can add it (the bits of ``y + bias``: the rounded output
+    plus the bias, rounded again), else None: a contiguous bf16 [n] tensor on x's device that
+    carries no gradient, tangent or batch dimension into the addition.  Saves the pass over the
+    output and its launch (eager, us a call: W6A8 333 x 5120 x 2688 42.5 -> 36.3, one MXFP8 row 22.7 ->
+    19.8)."""
+    if bias is None or type(bias) not in (torch.Tensor, torch.nn.Parameter):
+        return None
+    if bias.dtype != torch.bfloat16 or tuple(bias.shape) != (n,) or bias.device != x.device:
+        return None
+    if bias.layout != torch.strided or not bias.is_contiguous() or (bias.requires_grad and torch.is_grad_enabled()):
+        return None
+    if not torch.compiler.is_compiling():
+        if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.is_functorch_wrapped_tensor(bias):
+            return None
+    return bias
 
 
 def logical_mxfp6_shape(weight: torch.Tensor) -> tuple[int, int]:
@@ -210,10 +230,11 @@ class Mxfp6LinearKernel(_Kernel):
             raise ValueError("MXFP6 requires BF16 activations")
         if x.numel() == 0:
             return x.new_empty((*x.shape[:-1], n))
+        inner = _epilogue_bias(bias, x, n)
         y = ops.mx_gemm_from_float(_flatten(x, k).contiguous(), layer.weight, layer.weight_scale, n,
-                                   layer.mxl_format, self.act_rule)
+                                   layer.mxl_format, self.act_rule, inner)
         y = y.reshape(*x.shape[:-1], n)
-        return y if bias is None else y + bias
+        return y if bias is inner else y + bias
 
 
 class BlockFp8LinearKernel(_Kernel):
@@ -253,9 +274,10 @@ class BlockFp8LinearKernel(_Kernel):
             raise ValueError("block-FP8 requires BF16 activations with matching K")
         if x.numel() == 0:
             return x.new_empty((*x.shape[:-1], n))
-        y = ops.block_fp8_from_float(_flatten(x, k).contiguous(), layer.weight, layer.mxl_block_scale, n)
+        inner = _epilogue_bias(bias, x, n)
+        y = ops.block_fp8_from_float(_flatten(x, k).contiguous(), layer.weight, layer.mxl_block_scale, n, inner)
         y = y.reshape(*x.shape[:-1], n)
-        return y if bias is None else y + bias
+        return y if bias is inner else y + bias
 
 
 _KERNELS = {
