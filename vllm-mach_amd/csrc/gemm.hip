@@ -566,7 +566,10 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   const bool stream_ok = stream_gemm_eligible(M, K, block);
   const bool wide_ok = wide_gemm_eligible(M, K) && (!block || K <= int64_t(128) * kWideBlockStages);
   const bool chunk_ok = !block && chunk_gemm_eligible(M, K, fmt);
-  const bool tiles_ok = !four_wave && M > 16 && wide_tiles_eligible(M, N, K, block);
+  // The 2 x 2-wave tiles are the automatic choice's; a call that sets a tile, split or wave field
+  // plans among the kernels those fields name (four waves side by side: M >= 64, K % 256 == 0).
+  const bool auto_tile = o.tile_n == 0 && o.splits == 0 && o.waves == 0 && o.tile_m == 0 && !o.hybrid;
+  const bool tiles_ok = !four_wave && auto_tile && M > 16 && wide_tiles_eligible(M, N, K, block);
   // Short K over few n-tiles: the generic kernel splits K over the waves of one workgroup
   // and writes bf16 directly, where the wide kernel needs a K split and its reduce to fill
   // the CUs.  Measured by a per-shape sweep over every kernel, tile and split (µs, generic
@@ -582,7 +585,7 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   // the plans of all eight m-tiles, which callers hold by name; a registered entry picks the tiles there.
   const bool chunk_pref = chunk_ok && chunk_gemm_preferred(M, N, K) && (M > 112 || !tiles_ok);
   const bool generic_pref =
-      (!block && M > 32 && M <= (four_wave ? 256 : 128) && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128) ||
+      (!block && M > 32 && M <= (tiles_ok ? 128 : 256) && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128) ||
       (M < 64 && K >= 1024 && N * K <= (K <= 2048 ? int64_t(12) << 20 : K <= 4096 ? int64_t(4) << 20 : 0));
   d.kernel = o.kernel == kAuto
                  ? (stream_ok                                        ? kStream
@@ -600,13 +603,13 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
     return true;
   }
   if (d.kernel == kWide) {
-    const bool auto_tile = o.tile_n == 0 && o.splits == 0 && o.waves == 0 && o.tile_m == 0 && !o.hybrid;
-    if (auto_tile && tiles_ok) {
+    if (tiles_ok) {
       d.wide = wide_tiles_config(M, N, K, block);
     } else {
       d.wide = wide_config(M, N, K, fmt, o);
       // no 2 x 2-wave block-FP8 tile of 256 columns
       if (d.wide.WM == 2 && ((block && d.wide.NT == 4) || !wide_tiles_eligible(M, N, K, block))) d.wide.WM = 1;
+      if (d.wide.MT == 4 && d.wide.NT == 1) return false;  // no four-wave tile of 64 x 64
     }
     d.need = wide_workspace_bytes(d.wide, M, N);
   } else if (d.kernel == kGeneric) {
