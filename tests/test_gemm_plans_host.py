@@ -2,7 +2,6 @@
 import pytest
 
 
-
 def _plan(M, N, K, fmt=0, block=0, **fields):
     from vllm_mach_amd import _lib
     return _lib.plan_name("mxl_gemm_plan_name", M, N, K, fmt, block, options=_lib.GemmOptions(**fields))
@@ -37,3 +36,31 @@ def test_a_tile_that_is_not_built_is_refused(pkg, kernel):
     with pytest.raises(_lib.MxlError):
         _plan(128, 17408, 5120, 2, kernel=kernel, tile_n=1, tile_m=4, splits=1)
     assert _plan(128, 17408, 5120, 2, kernel=kernel, tile_n=1, tile_m=8, splits=1).startswith("gemm_wide_kernel<2,8,1")
+
+
+GENERIC, WIDE = "gemm_kernel<", "gemm_wide_kernel<"
+
+
+@pytest.mark.parametrize("M,N,K,block,kernel", [
+    # up to 32 rows: a workgroup of 16 columns per CU (two at a short K)
+    (17, 2672, 3072, 0, GENERIC), (32, 4096, 9088, 0, GENERIC), (32, 4097, 9088, 0, WIDE), (32, 4096, 9216, 0, WIDE),
+    (32, 1040, 8192, 0, GENERIC), (32, 1040, 8320, 0, WIDE), (32, 1024, 8320, 0, GENERIC),
+    (17, 512, 896, 0, GENERIC), (17, 512, 768, 0, WIDE), (31, 8192, 2048, 0, GENERIC), (31, 8193, 2048, 0, WIDE),
+    # 33 to 64 rows: 32 rows by 32 columns; past K = 4096 only where its workgroups do not split K, past
+    # 4608 only where the row groups share an XCD (a multiple of eight column groups)
+    (33, 4096, 4096, 0, GENERIC), (33, 4097, 4096, 0, WIDE), (64, 2048, 4608, 0, GENERIC), (64, 2016, 4608, 0, WIDE),
+    (64, 2080, 4608, 0, GENERIC), (64, 2080, 4736, 0, WIDE), (64, 2304, 7424, 0, GENERIC), (64, 2304, 7552, 0, WIDE),
+    # more: 64 rows by 16 columns
+    (65, 2048, 4096, 0, GENERIC), (65, 2049, 4096, 0, WIDE), (65, 2048, 4352, 0, GENERIC), (65, 2032, 4352, 0, WIDE),
+    (65, 2048, 4480, 0, WIDE), (640, 400, 2176, 0, GENERIC), (641, 256, 3200, 0, WIDE), (1280, 192, 3072, 0, GENERIC),
+    (1281, 128, 2176, 0, WIDE),
+    # block-FP8
+    (32, 4096, 4608, 1, GENERIC), (32, 4096, 4736, 1, WIDE), (64, 4096, 4352, 1, GENERIC), (64, 4064, 4352, 1, WIDE),
+    (64, 4064, 2176, 1, GENERIC), (65, 128, 2176, 1, WIDE), (17, 8192, 2048, 1, WIDE),
+])
+def test_one_round_of_the_generic_kernel(pkg, M, N, K, block, kernel):
+    assert _plan(M, N, K, 0, block).startswith(kernel)
+    if kernel == GENERIC:
+        assert not _plan(M, N, K, 0, block).endswith("reduce8_kernel") or K > 4096
+    if not block:
+        assert _plan(M, N, K, 2).startswith(kernel) and _plan(M, N, K, 3).startswith(kernel)
