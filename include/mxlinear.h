@@ -243,8 +243,10 @@ int mxl_mx_gemm_ex(const void* a, const void* sa, int64_t M, const void* w_tiled
  * so the call needs no workspace argument.  No counterpart in the reference: for
  * callers that cannot allocate (HIP graph capture, tight serving loops).  The
  * plan (kernel, tile, split) is mxl_mx_gemm's, so the result is bit-identical to
- * mxl_mx_gemm with a large enough workspace; a shape whose plan needs more
- * scratch than the array holds returns MXL_EINVAL.  `stream` must belong to the
+ * mxl_mx_gemm with a large enough workspace; where the partials of a K split of the
+ * 2 x 2-wave tiles exceed the array, the split runs on a part of the output at a time.
+ * A shape whose plan without those tiles (options.waves = 4 where they are planned)
+ * needs more scratch than the array holds returns MXL_EINVAL.  `stream` must belong to the
  * current device.  All calls on one GPU share the array: calls that overlap on
  * one GPU (concurrent streams) race; every call overwrites what it reads. */
 int64_t mxl_noalloc_scratch_bytes(void);

@@ -141,21 +141,26 @@ def test_tiles_read_swizzled_scales(pkg, oracle_mod, dev, M, N, K):
     assert torch.equal(got[0], got[1])
 
 
-def test_noalloc_takes_a_plan_past_its_scratch(pkg, oracle_mod, dev):
-    """A shape whose plan splits K past the no-allocation scratch, though the four-wave plan
-    fits it (so the entry point takes the shape): runs whole-K."""
+@pytest.mark.parametrize("M,N,K,fmt,bias", [
+    (200, 9216, 32768, 0, False), (768, 4096, 17408, 0, False), (1500, 2040, 17408, 2, True),  # parts of the columns
+    (30000, 250, 17408, 3, True),                                                              # one n-block: of the rows
+])
+def test_noalloc_takes_a_plan_past_its_scratch(pkg, dev, M, N, K, fmt, bias):
+    """Shapes whose plan splits K past the no-allocation scratch, though the plan without the 2 x 2-wave
+    tiles fits it (so the entry point takes them): the bits of mxl_mx_gemm with a workspace."""
     from vllm_mach_amd import _lib
-    M, N, K, fmt = 200, 9216, 32768, 0
     assert _lib.query("mxl_gemm_workspace_bytes_ex", M, N, K, fmt, 0, None) > _lib.query("mxl_noalloc_scratch_bytes")
-    codes = torch.randint(0, 0x70, (N, K), dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
-    scales = torch.randint(118, 122, (N, K // 32), dtype=torch.uint8, device=dev)
-    w, sw = pkg.ops.pack_weight(codes, scales, fmt)
-    a, sa = torch.ops.mach_amd.quantize_mxfp8(_act(M, K, 3).to(dev), 0)
+    g = torch.Generator(device=dev).manual_seed(M)
+    width = K if fmt == 0 else K * 3 // 4
+    codes = torch.randint(0, 0x70 if fmt == 0 else 256, (N, width), generator=g, dtype=torch.uint8, device=dev)
+    scales = torch.randint(118, 122, (N, K // 32), generator=g, dtype=torch.uint8, device=dev)
+    w, sw = pkg.ops.pack_weight(codes.view(torch.float8_e4m3fn) if fmt == 0 else codes, scales, fmt)
+    a, sa = torch.ops.mach_amd.quantize_mxfp8(torch.randn(M, K, generator=g, device=dev).bfloat16(), 0)
+    b = torch.randn(N, generator=g, device=dev).bfloat16() if bias else None
     out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-    _lib.call("mxl_mx_gemm_noalloc", a.data_ptr(), sa.data_ptr(), M, w.data_ptr(), sw.data_ptr(), N, K, fmt, None,
-              out.data_ptr(), N, torch.cuda.current_stream(dev).cuda_stream)
-    ref = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, None)
-    _check(out.float().cpu().numpy(), ref.float().cpu().numpy())
+    _lib.call("mxl_mx_gemm_noalloc", a.data_ptr(), sa.data_ptr(), M, w.data_ptr(), sw.data_ptr(), N, K, fmt,
+              None if b is None else b.data_ptr(), out.data_ptr(), N, torch.cuda.current_stream(dev).cuda_stream)
+    assert torch.equal(out, torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, fmt, b))
 
 
 @pytest.mark.parametrize("N,K,fmt,gathered", [(200, 128, 2, False), (384, 1152, 3, True), (264, 2048, 0, True)])

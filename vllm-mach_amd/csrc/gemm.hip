@@ -651,9 +651,36 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   return true;
 }
 
+// A K split of the 2 x 2-wave tiles whose partials do not fit `bytes` (at least one tile's do), on as
+// many n-blocks at a time as do (or, where one n-block's do not, m-blocks of it): each slab's split
+// launch and reduce follow the one before on the stream, so the partials are free again and every
+// output is the sum that one launch of the whole plan writes.  MX weights, logical activation scales.
+static hipError_t launch_wide_slabs(int fmt, const WideConfig& c, const GemmParams& p, int64_t bytes, hipStream_t s) {
+  const int64_t bm = 16 * c.MT, bn = 64 * c.NT, mblocks = (p.M + bm - 1) / bm;
+  const int64_t fit = bytes / (bm * bn * 4 * c.S);  // tiles whose partials fit
+  const int64_t rows = fit < mblocks ? fit * bm : p.M, cols = fit < mblocks ? bn : fit / mblocks * bn;
+  for (int64_t n0 = 0; n0 < p.N; n0 += cols)
+    for (int64_t m0 = 0; m0 < p.M; m0 += rows) {
+      GemmParams q = p;
+      q.M = p.M - m0 < rows ? p.M - m0 : rows;
+      q.N = p.N - n0 < cols ? p.N - n0 : cols;
+      q.a = p.a + m0 * p.lda;
+      q.sa = static_cast<const uint8_t*>(p.sa) + m0 * (p.K / 32);
+      q.w = p.w + n0 / 16 * p.KT * tile_chunks(fmt) * 1024;
+      q.sw = static_cast<const uint8_t*>(p.sw) + n0 / 16 * p.KT * 256;
+      q.out = p.out + m0 * p.ldc + n0;
+      if (p.bias) q.bias = p.bias + n0;
+      const hipError_t e = launch_gemm_wide(fmt, false, c, q, 0, s);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
+}
+
+// (slabs: without room for a K split of the 2 x 2-wave tiles, run it slab by slab instead of whole-K)
 static int gemm_common(const void* a, const void* sa, int64_t M, const void* w_tiled, const void* sw, int64_t N,
                        int64_t K, int fmt, bool block, const void* bias, void* out, int64_t ldc, void* workspace,
-                       int64_t workspace_bytes, const GemmOptions& o, void* stream, const char* who) {
+                       int64_t workspace_bytes, const GemmOptions& o, void* stream, const char* who,
+                       bool slabs = false) {
   MXL_CHECK_ARG(M >= 0 && N > 0 && K > 0 && K % 128 == 0, "%s: need N > 0, K %% 128 == 0 (M=%lld N=%lld K=%lld)", who,
                 (long long)M, (long long)N, (long long)K);
   MXL_CHECK_ARG(ldc >= N, "%s: ldc < N", who);
@@ -692,13 +719,14 @@ static int gemm_common(const void* a, const void* sa, int64_t M, const void* w_t
     e = launch_gemm_chunk(fmt, p, s);
   } else if (d.kernel == kWide) {
     WideConfig wc = d.wide;
-    if (!room) {
+    const bool cut = !room && slabs && wc.WM == 2 && wc.S > 1;
+    if (!room && !cut) {
       wc = WideConfig{wc.NT, 1, (K + kTileK - 1) / kTileK};  // no room: skip the K split
       wc.MT = d.wide.MT;
       wc.WM = d.wide.WM;
     }
     p.S = wc.S;
-    e = launch_gemm_wide(fmt, block, wc, p, 0, s);
+    e = cut ? launch_wide_slabs(fmt, wc, p, workspace_bytes, s) : launch_gemm_wide(fmt, block, wc, p, 0, s);
   } else {
     GemmConfig c = d.gen;
     if (!room) c.S = 1;
@@ -843,8 +871,8 @@ extern "C" int mxl_mx_gemm_noalloc(const void* a, const void* sa, int64_t M, con
   MXL_CHECK_ARG(M >= 0 && N > 0 && K > 0 && K % 128 == 0, "%s: need N > 0, K %% 128 == 0 (M=%lld N=%lld K=%lld)", who,
                 (long long)M, (long long)N, (long long)K);
   if (M == 0) return MXL_OK;
-  // The split-K partials of the four-wave plan must fit the scratch (the shapes this entry
-  // point takes); where the plan mxl_mx_gemm makes needs more, it runs without its K split.
+  // The shapes this entry point takes: those whose plan without the 2 x 2-wave tiles fits the scratch.
+  // The plan that runs is mxl_mx_gemm's; a K split of its 2 x 2-wave tiles that needs more runs in slabs.
   DensePlan d;
   if (!plan_dense_as(M, N, K, w_fmt, false, with_override(M, N, K, w_fmt, false, GemmOptions()), d, true)) {
     set_error("%s: no kernel runs this shape (M=%lld, K=%lld)", who, (long long)M, (long long)K);
@@ -866,7 +894,7 @@ extern "C" int mxl_mx_gemm_noalloc(const void* a, const void* sa, int64_t M, con
   const int rc = scratch_address(who, &ws);
   if (rc != MXL_OK) return rc;
   return gemm_common(a, sa, M, w_tiled, sw_tiled, N, K, w_fmt, false, bias, out, ldc, ws, kNoAllocScratchBytes,
-                     GemmOptions(), stream, who);
+                     GemmOptions(), stream, who, true);
 }
 
 static int swiglu_row_common(const void* gate_up, int64_t M, int64_t K, int rule, const void* w_tiled,
