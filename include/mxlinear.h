@@ -222,7 +222,8 @@ int mxl_mx_gemm_dual_ex(const void* hi, const void* s_hi, const void* res, const
 
 /* MX block-scaled GEMM: y[M, N] (bf16, row stride ldc) = A . W^T, A = E4M3
  * codes [M, K] + E8M0 [M, K/32]; W tiled (fmt 0/2/3); bias bf16 [N] or NULL
- * (added after the bf16 rounding, as y + bias in bf16).  Replaces
+ * (added after the bf16 rounding, as y + bias in bf16).  Scales that are not 4-byte
+ * aligned run on the generic kernel wherever the plan is a wide one.  Replaces
  * mxfp8_sm120::gemm (src/vllm_mach/mxfp6/dense_mxfp8.py:86,
  * src/vllm_mach/mxfp8/native_backend.py:77-89) and mxfp6::gemm_w6a8_pdl
  * (src/vllm_mach/mxfp6/ar_norm.py:144-147). */

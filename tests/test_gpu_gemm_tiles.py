@@ -185,3 +185,28 @@ def test_grouped_tiles(pkg, dev, monkeypatch, N, K, fmt, gathered):
         got.append(torch.ops.mach_amd.grouped_gemm(*args).float().cpu().numpy())
     assert (got[0] == got[1]).all()  # whole-K sums are the same chain of MFMAs
     _check(got[0], got[2])
+
+
+def _byte_past(t):
+    """The same bytes one past a dword boundary."""
+    flat = torch.empty(t.numel() + 4, dtype=torch.uint8, device=t.device)
+    flat[1:1 + t.numel()] = t.reshape(-1).view(torch.uint8)
+    return flat[1:1 + t.numel()].view(t.shape)
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 4352, 5248), (333, 2048, 2688), (700, 4096, 2560)])
+def test_scales_at_any_byte(pkg, oracle_mod, dev, M, N, K):
+    """The tiles copy activation scales by the dword: scales that are not dword-aligned run on the
+    generic kernel (the same bits), dense and grouped."""
+    from vllm_mach_amd import _lib
+    ops = pkg.ops
+    a, sa, w, sw = _mx(pkg, oracle_mod, dev, M, N, K, 2)
+    assert _lib.plan_name("mxl_gemm_plan_name", M, N, K, 2, 0).startswith("gemm_wide_kernel<")
+    with ops.tuning(kernel=ops.KERNEL_GENERIC):
+        ref = torch.ops.mach_amd.mx_gemm(a, sa, w, sw, N, K, 2, None)
+    assert torch.equal(torch.ops.mach_amd.mx_gemm(a, _byte_past(sa), w, sw, N, K, 2, None), ref)
+    offsets = torch.tensor([0, M], device=dev)
+    with ops.tuning(kernel=ops.KERNEL_GENERIC):
+        ref = torch.ops.mach_amd.grouped_gemm(a, sa, None, 1, offsets, M, w, sw, N, K, 2)
+    assert _lib.plan_name("mxl_grouped_plan_name", M, 1, K, 2, 0, 0).startswith("gemm_wide_kernel<")
+    assert torch.equal(torch.ops.mach_amd.grouped_gemm(a, _byte_past(sa), None, 1, offsets, M, w, sw, N, K, 2), ref)

@@ -484,6 +484,10 @@ static GemmOptions options_of(const void* opts) {
 
 static bool default_epilogue(const GemmOptions& o) { return o.out_dtype == kOutBf16 && o.alpha == 1.0f; }
 
+// The wide tiles copy scales from global memory straight to LDS, by the dword and by four, which
+// needs dword-aligned memory; the other kernels load them into registers, at any alignment.
+static bool dword_aligned(const void* sa, const void* sw) { return (((uintptr_t)sa | (uintptr_t)sw) & 3) == 0; }
+
 // The dense kernel and split a call runs with (shared by the launch and the workspace
 // query, so that the bytes the query reports are the bytes the launch uses).
 struct DensePlan {
@@ -694,6 +698,11 @@ static int gemm_common(const void* a, const void* sa, int64_t M, const void* w_t
   if (!plan_dense(M, N, K, fmt, block, o, d)) {
     set_error("%s: kernel %d does not run (M=%lld, K=%lld)", who, o.kernel, (long long)M, (long long)K);
     return MXL_EUNSUPPORTED;
+  }
+  if (d.kernel == kWide && !dword_aligned(sa, sw)) {
+    d.kernel = kGeneric;
+    d.gen = choose_config(M, N, K);
+    d.need = d.gen.S > 1 ? (int64_t)d.gen.S * M * N * 4 : 0;
   }
   GemmParams p{};
   p.a = (const uint8_t*)a; p.sa = sa; p.w = (const uint8_t*)w_tiled; p.sw = sw;
@@ -1383,7 +1392,7 @@ static int grouped_common(const void* a, const void* sa, int64_t a_rows, const i
   MXL_CHECK_ARG(default_epilogue(o), "mxl_grouped_gemm: bf16 output without scaling only");
   const GroupedPlan gp = plan_grouped(a_rows, num_experts, routed_rows, K, w_fmt, o);
   const int stream_mt = gp.stream_mt;
-  if (gp.kernel == kWide && wide_tiles_eligible(a_rows, N, K, false)) {
+  if (gp.kernel == kWide && wide_tiles_eligible(a_rows, N, K, false) && dword_aligned(sa, sw_tiled)) {
     // enough rows per expert on average for 128-row blocks: the wide kernel
     GemmParams p{};
     p.a = (const uint8_t*)a; p.sa = sa; p.w = (const uint8_t*)w_tiled; p.sw = sw_tiled;
