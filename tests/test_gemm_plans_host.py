@@ -64,3 +64,29 @@ def test_one_round_of_the_generic_kernel(pkg, M, N, K, block, kernel):
         assert not _plan(M, N, K, 0, block).endswith("reduce8_kernel") or K > 4096
     if not block:
         assert _plan(M, N, K, 2).startswith(kernel) and _plan(M, N, K, 3).startswith(kernel)
+
+
+def test_kept_plans_are_the_plans_of_their_sizes(pkg):
+    """More shapes than a thread keeps plans for, from one thread and from several, and around a registered
+    entry: a kept plan answers for its own sizes, format and mode only."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from vllm_mach_amd import _lib
+    shapes = [(M, N, K, fmt, block) for M in (24, 96, 333, 2048) for N in (512, 2560, 17408) for K in (1024, 2688, 9216)
+              for fmt, block in ((0, 0), (2, 0), (3, 0), (0, 1))]
+
+    def plans(order):
+        return {s: (_plan(*s), _lib.query("mxl_gemm_workspace_bytes_ex", *s, None)) for s in order}
+
+    one_by_one = {}
+    for s in shapes:  # a new thread has kept nothing
+        with ThreadPoolExecutor(1) as pool:
+            one_by_one[s] = pool.submit(plans, [s]).result()[s]
+    with ThreadPoolExecutor(4) as pool:
+        for got in pool.map(plans, [shapes, shapes[::-1], shapes * 2, shapes[::3] + shapes]):
+            assert all(one_by_one[s] == p for s, p in got.items())
+    s = (333, 2560, 2688, 2, 0)
+    _lib.call("mxl_set_gemm_config", *s, _lib.options_ptr(_lib.GemmOptions(kernel=2)))
+    assert _plan(*s).startswith("gemm_kernel<2,") != one_by_one[s][0].startswith("gemm_kernel<2,")
+    _lib.call("mxl_clear_gemm_configs")
+    assert plans([s])[s] == one_by_one[s]

@@ -589,8 +589,30 @@ static bool generic_round(int64_t M, int64_t N, int64_t K, bool block) {
   return !block && (M <= 640 ? K <= (shared ? 4352 : 4096) : M <= 1280 && K <= 3072);
 }
 
+// An automatic plan is a function of the sizes, the weight and the CUs, and a call asks for it up to four
+// times (the workspace query over the formats, then the launch), so each thread keeps the last of
+// each of 128 slots: a serving loop's layer shapes stay (a workspace query over two alternating
+// layers of 333 rows takes 0.64 us, planned anew each time 1.7).
 static bool plan_dense(int64_t M, int64_t N, int64_t K, int fmt, bool block, const GemmOptions& o, DensePlan& d) {
-  return plan_dense_as(M, N, K, fmt, block, with_override(M, N, K, fmt, block, o), d);
+  const GemmOptions r = with_override(M, N, K, fmt, block, o);
+  if (!tuning_auto(r)) return plan_dense_as(M, N, K, fmt, block, r, d);
+  struct Kept {
+    int64_t M = 0, N = 0, K = 0, cus = 0;
+    int fmt = 0, block = 0;
+    DensePlan d;
+  };
+  static thread_local Kept kept[128];
+  constexpr uint64_t mix = 0x9E3779B97F4A7C15ull;
+  const uint64_t h = (((uint64_t)M * mix + (uint64_t)N) * mix + (uint64_t)K) * mix + (uint64_t)(2 * fmt + block);
+  Kept& k = kept[h * mix >> 57];
+  const int64_t cus = cu_count();
+  if (k.M != M || k.N != N || k.K != K || k.cus != cus || k.fmt != fmt || k.block != (int)block) {
+    DensePlan fresh;
+    if (!plan_dense_as(M, N, K, fmt, block, r, fresh)) return false;
+    k = Kept{M, N, K, cus, fmt, block, fresh};
+  }
+  d = k.d;
+  return true;
 }
 
 // (four_wave: the plan of the four-wave tiles alone, whatever the 2 x 2-wave ones would do)

@@ -798,7 +798,7 @@ bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
 }
 
 // Tile, split and hybrid of the 2 x 2-wave kernels by the time model.
-static WideConfig wide_tiles_choice(int64_t M, int64_t N, int64_t K, bool block) {
+WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
   const int64_t KT = (K + kTileK - 1) / kTileK, T = (K + 127) / 128, cus = cu_count();
   const double out = 2.0 * M * N / kTileOutBytesPerUs;
   WideConfig best{2, 1, KT};
@@ -840,20 +840,6 @@ static WideConfig wide_tiles_choice(int64_t M, int64_t N, int64_t K, bool block)
   }
   best.WM = 2;
   return best;
-}
-
-// The choice is a function of the sizes; a call asks for it up to four times (the workspace query
-// over the formats, then the launch), so each thread keeps its last two (0.6 us each).
-WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
-  struct Last {
-    int64_t M, N, K, cus;
-    WideConfig c;
-  };
-  static thread_local Last last[2] = {};
-  Last& l = last[block];
-  const int64_t cus = cu_count();
-  if (l.M != M || l.N != N || l.K != K || l.cus != cus) l = Last{M, N, K, cus, wide_tiles_choice(M, N, K, block)};
-  return l.c;
 }
 
 int64_t wide_workspace_bytes(const WideConfig& c, int64_t M, int64_t N) {
