@@ -56,6 +56,8 @@ TILES = [
     (1500, 18432, 512, 0, "16,4", False),  # one super-tile; quarters
     (700, 18400, 2560, 2, "16,4", False),  # N % 256 = 224
     (2000, 9000, 1280, 3, "16,4", False),  # quarters of 32 tiles: 80 rows, 40 columns of the last
+    (749, 6408, 1024, 0, "8,2", False),    # quarters of 50 tiles beside the one round of whole ones
+    (1290, 3208, 1664, 3, "8,2", False),   # of 30, an odd count of slices: 10 rows, 8 columns of the last
 ]
 
 
@@ -82,6 +84,7 @@ def test_mx_tiles(pkg, oracle_mod, dev, monkeypatch, M, N, K, fmt, tile, split):
     (130, 18432, 640, "4,2", False),
     (300, 18432, 2560, "8,2", False),
     (1090, 7552, 1280, "8,2", False),   # quarters of 19 tiles, 2 rows of the last
+    (793, 5504, 1152, "8,2", False),    # of 45 tiles beside the one round
 ])
 def test_block_fp8_tiles(pkg, dev, monkeypatch, M, N, K, tile, split):
     ops = pkg.ops

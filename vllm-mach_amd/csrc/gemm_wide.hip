@@ -759,11 +759,13 @@ WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptio
 
 // ---- 2 x 2-wave tiles
 //
-// Time model, fitted to a sweep of every tile and split over 184 dense shapes (M 17..2048, N
-// 256..18432, K 512..17408, MXFP8, MXFP6 and block-FP8 weights rotated out of the caches): a launch
-// costs its fixed time, the stages of the fullest CU, its output, which nothing overlaps in the last
-// round, and its operands from HBM (at 10.6 TB/s; the same for every choice, so left out below).  Its pick runs within 0.9 % of the best of them on average
-// (the farthest: 722 x 11264 x 896 21.0 us against 18.1, 561 x 1792 x 17408 38.4 against 32.9).
+// Time model, fitted to a sweep of every tile and split over dense shapes of 17 to 4096 rows with
+// MXFP8, MXFP6 and block-FP8 weights rotated out of the caches: a launch costs its fixed time, the
+// stages of the fullest CU, and its output, which nothing overlaps in the last round.  What all
+// choices share is left out (the operands' way from memory), so it is some 7 % low on average.  The
+// plans of 1103 shapes run within 1.0 % of the best tile and split on average (the farthest of its
+// picks: 200 x 16640 x 512 12.0 us against 9.0, 3912 x 2208 x 512 15.5 against 12.1, 1470 x 2816 x 5760
+// 40.4 against 34.0).
 struct TileCost {
   int MT, NT, resident;   // tile, workgroups per CU
   double fixed, stage;    // us: of the launch, of a K128 stage on one CU
@@ -777,19 +779,32 @@ constexpr double kTileBlockAlone = 1.06, kTileBlockShared = 0.874;
 constexpr double kTileGap = 0.5;                  // a further round's start on a CU, us
 constexpr double kTileReduce = 3.2;               // the split reduce's launch, us
 constexpr double kTileOutBytesPerUs = 2.3e6, kTilePartialBytesPerUs = 6.1e6;
-// the few tiles of a hybrid's remainder: their partials stay in the caches
-constexpr double kTileRemainderBytesPerUs = 8.9e6;
+// A hybrid (one round of 128 x 128 tiles whole, the rest split in K beside them): its fixed time and
+// reduce, us; a whole tile's stage, at two stages in flight since the units share its CU's LDS, MX and
+// block-FP8; a unit's stage; the units' partials.  (Fitted to 236 of them, 2 us rms.)
+constexpr double kHybridFixed = 9.4, kHybridStage = 0.52, kHybridBlockStage = 0.61, kHybridUnitStage = 0.376;
+constexpr double kHybridBytesPerUs = 7.6e6;
+// the same where the hybrid stays, below: as its parts would cost alone
+constexpr double kHybridKeptBytesPerUs = 8.9e6;
 
 // Tiles of a partly filled last round that run as four quarters each, so that their K walk ends
 // sooner: where the quarters' stages on the fullest CU are clearly fewer than the tile's (W6A8
 // 1024 x 17408 x 5120 in 256 x 256 tiles, 16 past a full round: 116.6 to 95.2 us; block-FP8 512 x
-// 18432 x 2560 in 128 x 128, 64 past 512: 44.2 to 37.1).  After at least one full round of
-// resident workgroups: with fewer tiles the hybrid below splits the remainder in K.
+// 18432 x 2560 in 128 x 128, 64 past 512: 44.2 to 37.1).  Tiles of two workgroups per CU have them
+// after one round of the CUs too, beside the whole tiles (MXFP8 749 x 6400 x 1024, 44 tiles past it:
+// 12.3 us, whole-K 15.1, hybrid 17.4; block-FP8 793 x 5504 x 2432, 45: 21.3, 25.2, 27.5).
 static int64_t wide_tail(const TileCost& t, int64_t tiles, int64_t cus) {
   const int64_t rem = tiles % cus;
-  if (t.quarter == 0 || tiles <= t.resident * cus || rem == 0) return 0;
+  if (t.quarter == 0 || tiles <= cus || rem == 0) return 0;
   return (double)((4 * rem + cus - 1) / cus) * t.quarter < 0.9 * t.stage ? rem : 0;
 }
+
+// Up to two blocks of 128 rows the weights' way from memory sets the pace, and over a long K the
+// hybrid's units end beside the whole tiles: MX from K = 5120 it runs even with the quarters or ahead
+// (160 / 256 x 16640 / 17408 x 5120 36.0 / 40.4 us against 39.7 / 40.3, 200 x 16640 x 8192 47.7 against
+// 53.7; 256 x 18432 x 4096 35.6 against 32.4).  Block-FP8 gives up 2 to 14 % there to keep the plan of
+// its gate_up layer, which is held by name (256 x 18432 x 2560 27.8 against 23.9).
+static bool hybrid_kept(int64_t M, int64_t K, bool block) { return M <= 256 && K >= (block ? 2560 : 5120); }
 
 bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
   // 32-bit operand offsets
@@ -801,6 +816,7 @@ bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
 WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
   const int64_t KT = (K + kTileK - 1) / kTileK, T = (K + 127) / 128, cus = cu_count();
   const double out = 2.0 * M * N / kTileOutBytesPerUs;
+  const bool kept = hybrid_kept(M, K, block);
   WideConfig best{2, 1, KT};
   double best_us = 1e300;
   for (const TileCost& t : kTileCosts) {
@@ -821,7 +837,7 @@ WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
       const int64_t per = (KT + s - 1) / s;
       if ((KT + per - 1) / per != s) continue;
       const int64_t stages = per * 4 < T ? per * 4 : T, n = (tiles * s + cus - 1) / cus;
-      const int64_t tail = s == 1 ? wide_tail(t, tiles, cus) : 0;
+      const int64_t tail = s == 1 && !(kept && tiles <= t.resident * cus) ? wide_tail(t, tiles, cus) : 0;
       double us = t.fixed;
       if (tail) us += work(n - 1, stages) + (4 * tail + cus - 1) / cus * stages * t.quarter + kTileGap;
       else us += work(n, stages);
@@ -829,14 +845,16 @@ WideConfig wide_tiles_config(int64_t M, int64_t N, int64_t K, bool block) {
       else us += kTileReduce + ((double)M * N * 8 * s + 2.0 * M * N) / kTilePartialBytesPerUs;
       take(us, WideConfig{t.NT, (int)s, per});
     }
-    // the hybrid after one full round only (after two it measured within 6 % of whole-K either
-    // way): block-FP8 256 x 18432 x 2560 27.5 us against 30.5 whole-K, W6A8 256 x 17408 x 5120 40.2
-    // against 54.1.  (Quarters for the remainder would take 24.3 and 40.3 there.)
+    // (after one full round only: after two it measured within 6 % of whole-K either way)
     WideConfig h{t.NT, 1, KT};
-    if (t.MT == 8 && t.NT == 2 && wide_hybrid(tiles, KT, cus, h) && h.dp_tiles == cus)
-      take(t.fixed + work(1, T) + h.kt2 * 4 * t.stage * (block ? kTileBlockShared : 1.0) + kTileReduce +
-               (double)(tiles - cus) * 128 * 128 * 8 * h.S2 / kTileRemainderBytesPerUs,
+    if (t.MT == 8 && t.NT == 2 && wide_hybrid(tiles, KT, cus, h) && h.dp_tiles == cus) {
+      const double units = h.kt2 * 4, bytes = (double)(tiles - cus) * 128 * 128 * 8 * h.S2;
+      take(kept ? t.fixed + work(1, T) + units * t.stage * (block ? kTileBlockShared : 1.0) + kTileReduce +
+                      bytes / kHybridKeptBytesPerUs
+                : kHybridFixed + T * (block ? kHybridBlockStage : kHybridStage) + units * kHybridUnitStage +
+                      bytes / kHybridBytesPerUs,
            h);
+    }
   }
   best.WM = 2;
   return best;
