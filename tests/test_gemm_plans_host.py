@@ -98,3 +98,9 @@ def test_a_part_round_of_tiles_runs_in_one_launch(pkg, M, N, K, block):
     """Up to 64 tiles of 128 x 128 past one round of the CUs: their quarters beside the whole tiles, not a K
     split and its reduce (2 to 5 us slower at each of these)."""
     assert _plan(M, N, K, 0, block) == f"gemm_wide_kernel<0,8,2,{'true' if block else 'false'},false,2>"
+
+
+@pytest.mark.parametrize("M", [65, 112, 113, 120, 127, 129])
+@pytest.mark.parametrize("N,K,fmt", [(4608, 2048, 2), (8192, 1920, 3), (17408, 1536, 0)])
+def test_tiles_take_the_rows_on_either_side_of_the_chunked_plan(pkg, M, N, K, fmt):
+    assert _plan(M, N, K, fmt).startswith(f"gemm_wide_kernel<{fmt},")

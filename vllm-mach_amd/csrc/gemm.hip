@@ -637,9 +637,10 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   // 5760 9.6 against 8.5); at 129 to 256 rows the tiles win (256 of 2048 x 2048 8.6 against 7.5).
   // It also keeps what generic_round below takes.
   // The chunked kernel beat the four-wave tiles; the 2 x 2-wave ones pass it wherever it was chosen
-  // (W6A8 4608 x 2048 at 72 / 96 / 128 rows 7.9 / 8.0 / 8.4 against 11.9 / 11.9 / 12.1).  It keeps
-  // the plans of all eight m-tiles, which callers hold by name; a registered entry picks the tiles there.
-  const bool chunk_pref = chunk_ok && chunk_gemm_preferred(M, N, K) && (M > 112 || !tiles_ok);
+  // (W6A8 4608 x 2048 at 72 / 113 / 128 rows 7.9 / 8.1 / 8.3 us against 11.9 / 12.1 / 12.0, 120 x 8192 x 1920
+  // 8.6 against 12.9; MXFP8 120 x 17408 x 1536 13.5 against 19.7).  At 128 rows its plan stays, which is
+  // held by name; a registered entry can name the four-wave tiles there (10.7).
+  const bool chunk_pref = chunk_ok && chunk_gemm_preferred(M, N, K) && (M == 128 || !tiles_ok);
   const bool generic_pref =
       (!block && M > 32 && M <= (tiles_ok ? 128 : 256) && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128) ||
       (M < 64 && K >= 1024 && N * K <= (K <= 2048 ? int64_t(12) << 20 : K <= 4096 ? int64_t(4) << 20 : 0)) ||
