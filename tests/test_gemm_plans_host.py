@@ -52,7 +52,8 @@ GENERIC, WIDE = "gemm_kernel<", "gemm_wide_kernel<"
     (64, 2080, 4608, 0, GENERIC), (64, 2080, 4736, 0, WIDE), (64, 2304, 7424, 0, GENERIC), (64, 2304, 7552, 0, WIDE),
     # more: 64 rows by 16 columns
     (65, 2048, 4096, 0, GENERIC), (65, 2049, 4096, 0, WIDE), (65, 2048, 4352, 0, GENERIC), (65, 2032, 4352, 0, WIDE),
-    (65, 2048, 4480, 0, WIDE), (640, 400, 2176, 0, GENERIC), (641, 256, 3200, 0, WIDE), (1280, 192, 3072, 0, GENERIC),
+    (65, 2048, 5376, 0, GENERIC), (65, 2048, 5504, 0, WIDE), (65, 1536, 5376, 0, GENERIC), (65, 1408, 4480, 0, WIDE),
+    (640, 400, 2176, 0, GENERIC), (641, 256, 3200, 0, WIDE), (1280, 192, 3072, 0, GENERIC),
     (1281, 128, 2176, 0, WIDE),
     # block-FP8
     (32, 4096, 4608, 1, GENERIC), (32, 4096, 4736, 1, WIDE), (64, 4096, 4352, 1, GENERIC), (64, 4064, 4352, 1, WIDE),

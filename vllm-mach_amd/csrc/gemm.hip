@@ -573,8 +573,9 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
 //     unsplit 0.84 to 0.95, up to 7424 shared 0.80 to 0.99 (otherwise 0.90 to 1.26); block-FP8 up to 4096
 //     0.79 to 1.05, up to 4352 shared 0.85 to 0.89 (past it 0.98 to 1.44)
 //   65 to 640 rows, MX: 2176 to 4096 0.80 to 1.06 (200 x 1024 x 3328 8.1 against 9.2), up to 4352 unsplit
-//     shared 0.89 to 0.99 (past it 0.91 to 1.67); up to 1280 rows 2176 to 3072 0.80 to 1.03 (past it up
-//     to 1.37).  Block-FP8 from 65 rows 1.03 to 1.17 and more.
+//     shared 0.89 to 0.99 (past it 0.91 to 1.67), up to 5376 shared by at least 3/4 of the CUs 0.91 to 1.04
+//     (256 x 1024 x 4480 9.8 against 10.6, 180 x 1280 x 5248 11.3 both, and one launch for two); up to 1280 rows
+//     2176 to 3072 0.80 to 1.03 (past it up to 1.37).  Block-FP8 from 65 rows 1.03 to 1.17 and more.
 // Two workgroups per CU are one round too at 17 to 32 rows and K = 1024 to 2048, MX: 0.87 to 0.97
 // (31 x 6656 x 1920 6.5 us against 7.5; with more of them 1.07 to 1.58).
 static bool generic_round(int64_t M, int64_t N, int64_t K, bool block) {
@@ -586,7 +587,7 @@ static bool generic_round(int64_t M, int64_t N, int64_t K, bool block) {
   if (groups > cus || K <= (!block && M <= 32 ? 768 : 2048)) return false;
   if (M <= 32) return K <= (block ? 4608 : unsplit || groups <= 64 ? 9088 : 8192);
   if (M <= 64) return K <= (block ? (shared ? 4352 : 4096) : shared ? 7424 : unsplit ? 4608 : 4096);
-  return !block && (M <= 640 ? K <= (shared ? 4352 : 4096) : M <= 1280 && K <= 3072);
+  return !block && (M <= 640 ? K <= (!shared ? 4096 : 4 * groups >= 3 * cus ? 5376 : 4352) : M <= 1280 && K <= 3072);
 }
 
 // An automatic plan is a function of the sizes, the weight and the CUs, and a call asks for it up to four
