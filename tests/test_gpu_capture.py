@@ -175,3 +175,31 @@ def test_warmup_then_capture_allocates_no_workspace(pkg, dev):
     assert after["retired_bytes"] == before["retired_bytes"]
     assert after["counts"].get("workspace_miss", 0) == before["counts"].get("workspace_miss", 0)
     assert "capture_cache_miss" not in after["counts"]
+
+
+def test_stream_handle_is_the_current_streams(pkg, dev):
+    """Default and other streams, nested, on another thread and under capture; devices with and without index."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from vllm_mach_amd._lib import stream_handle
+
+    def check():
+        for d in (dev, torch.device("cuda")):
+            assert stream_handle(d) == torch.cuda.current_stream(d).cuda_stream
+
+    check()
+    a, b = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    with torch.cuda.stream(a):
+        check()
+        assert stream_handle(dev) == a.cuda_stream
+        with torch.cuda.stream(b):
+            check()
+        with ThreadPoolExecutor(1) as pool:  # a stream is current on its own thread
+            pool.submit(check).result()
+        check()
+    x = torch.zeros(4, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a):
+        x += 1
+        check()
+    check()

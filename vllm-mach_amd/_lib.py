@@ -153,4 +153,6 @@ def plan_name(fn: str, *args, options: "GemmOptions | None" = None) -> str:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of ``device``'s current stream (``torch.cuda.current_stream(device).cuda_stream``
+    without the stream object, 2.0 us: an eager layer call asks for it two to six times)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
