@@ -81,7 +81,8 @@ struct TileB<kE3M2> { typedef v6i type; };
 // accumulator registers live the compiler's allocator finds no room to rename one, and moves
 // whole tiles between register files instead (measured on its output: several hundred moves
 // and spills per stage).  The caller keeps two instructions between a VALU write of an
-// operand and its use, and waits out the last MFMA before it reads an accumulator.
+// operand and its use, and waits out the last MFMA before it or the compiler reads an accumulator
+// (tests/test_mfma_hazards_host.py scans the built code for both).
 template <int FMT, int J>
 __device__ __forceinline__ void tile_mfma(v4f& c, const typename TileB<FMT>::type& w, const v8i& a, uint32_t sw,
                                           uint32_t sa) {
@@ -488,6 +489,9 @@ __device__ __forceinline__ void tile_gemm(const GemmParams& p, const TileWork& w
     const int one = cur + L::STAGE < ring ? cur + L::STAGE : 0, two = one + L::STAGE < ring ? one + L::STAGE : 0;
     stage(Slice<0>{}, Slice<left>{}, 2 * pr, cur, one);
     stage(Slice<1>{}, Slice<left ? left - 1 : 0>{}, 2 * pr + 1, one, two);
+    // 64 x 64 tiles: the compiler moves the accumulators after the loop, 17 states after the last MFMA whose
+    // result takes 20
+    if constexpr (!BLOCK && MTW * NTW == 4) asm volatile("s_nop 2");
     cur = two;
   };
   const int last = end >> 1;  // pairs 2 kb .. last - 1; the copies end in the final one or two
