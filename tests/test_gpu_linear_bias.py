@@ -39,3 +39,30 @@ def test_bias_bits(pkg, dev, kind, n, k, M):
         assert torch.equal(got.isnan(), want.isnan())
     method.apply(layer, x, grad).float().nan_to_num().sum().backward()
     assert grad.grad is not None
+
+
+@pytest.mark.parametrize("kind,n,k", [("mxfp8", 640, 1024), ("mxfp6", 520, 2688), ("block", 512, 1152)])
+@pytest.mark.parametrize("M", [1, 40])
+def test_bias_under_transforms(pkg, dev, kind, n, k, M):
+    """A bias that carries a tangent, a batch dimension or a gradient of a transform into the addition, or is
+    traced, is added as torch does it."""
+    method, layer = _layer(pkg, dev, kind, n, k)
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, k, generator=g).bfloat16().to(dev)
+    biases = torch.randn(3, n, generator=g).bfloat16().to(dev)
+    bias, tangent = biases[0], biases[1]
+    y = method.apply(layer, x, None)
+    call = lambda b: method.apply(layer, x, b)  # noqa: E731
+    assert torch.equal(torch.func.vmap(call)(biases), y + biases[:, None])
+    out, t = torch.func.jvp(call, (bias,), (tangent,))
+    assert torch.equal(out, y + bias) and torch.equal(t, tangent.expand(M, n))
+    with torch.autograd.forward_ad.dual_level():
+        dual = call(torch.autograd.forward_ad.make_dual(bias, tangent))
+        out, t = torch.autograd.forward_ad.unpack_dual(dual)
+        assert torch.equal(out, y + bias) and torch.equal(t, tangent.expand(M, n))
+    ones = torch.func.grad(lambda b: call(b).float().sum())(bias)
+    assert torch.equal(ones, torch.full_like(bias, M))
+    traced = torch.compile(call, fullgraph=M > 16, backend="eager")  # (up to 16 rows the route asks the library)
+    assert torch.equal(traced(bias), y + bias)
+    with torch.no_grad():
+        assert torch.equal(call(torch.nn.Parameter(bias)), y + bias)

@@ -37,3 +37,25 @@ def test_route_sort_with_dropped_ids(pkg, oracle_mod, dev, R, E):
     n = int(ro[-1])
     assert np.array_equal(o.cpu().numpy(), ro) and np.array_equal(inv.cpu().numpy(), rinv)
     assert np.array_equal(s.cpu().numpy()[:n], rs[:n])
+
+
+@pytest.mark.parametrize("T,E,topk", [(8, 256, 8), (40, 300, 4), (1030, 64, 2)])
+@pytest.mark.parametrize("renorm", [True, False])
+def test_router_orders_nan_logits_by_their_bits(pkg, oracle_mod, dev, T, E, topk, renorm):
+    """A NaN without sign lies above every logit, one with it below, an all-ones one lowest of all (its order key
+    is 0, what a taken logit's becomes): ids and tables by that order, weights of the other rows as without."""
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, E, generator=g)
+    bits = x.view(torch.int32)
+    bits[1, 3], bits[1, E - 1] = 0x7FC00000, 0x7F800001
+    bits[2, ::2] = -1
+    bits[3] = -1
+    bits[4, 0], bits[4, 5] = -0x400000, 0x7FFFFFFF               # 0xFFC00000
+    w, ids, s, o, inv = torch.ops.mach_amd.moe_router(x.to(dev), topk, renorm)
+    rw, rids, rs, ro, rinv = oracle_mod.moe_router(x.numpy(), topk, renorm)
+    assert np.array_equal(ids.cpu().numpy(), rids)
+    assert np.array_equal(o.cpu().numpy(), ro) and np.array_equal(s.cpu().numpy(), rs)
+    assert np.array_equal(inv.cpu().numpy(), rinv)
+    plain = [0] + list(range(5, T))
+    assert np.abs(w.double().cpu().numpy()[plain] - rw[plain]).max() <= 4e-6
+    assert bool(w[1].isnan().all())
