@@ -41,30 +41,36 @@ def test_a_tile_that_is_not_built_is_refused(pkg, kernel):
 GENERIC, WIDE = "gemm_kernel<", "gemm_wide_kernel<"
 
 
-@pytest.mark.parametrize("M,N,K,block,kernel", [
+@pytest.mark.parametrize("M,N,K,block,mxfp8,mxfp6", [
     # up to 32 rows: a workgroup of 16 columns per CU (two at a short K)
-    (17, 2672, 3072, 0, GENERIC), (32, 4096, 9088, 0, GENERIC), (32, 4097, 9088, 0, WIDE), (32, 4096, 9216, 0, WIDE),
-    (32, 1040, 8192, 0, GENERIC), (32, 1040, 8320, 0, WIDE), (32, 1024, 8320, 0, GENERIC),
-    (17, 512, 896, 0, GENERIC), (17, 512, 768, 0, WIDE), (31, 8192, 2048, 0, GENERIC), (31, 8193, 2048, 0, WIDE),
+    (17, 2672, 3072, 0, GENERIC, GENERIC), (32, 4096, 8192, 0, GENERIC, GENERIC), (32, 4097, 8192, 0, WIDE, WIDE),
+    (32, 4096, 9088, 0, WIDE, GENERIC), (32, 4096, 9216, 0, WIDE, WIDE), (32, 1040, 8192, 0, GENERIC, GENERIC),
+    (32, 1040, 8320, 0, WIDE, WIDE), (32, 1024, 8320, 0, WIDE, GENERIC), (17, 512, 896, 0, GENERIC, GENERIC),
+    (17, 512, 768, 0, WIDE, WIDE), (31, 8192, 2048, 0, GENERIC, GENERIC), (31, 8193, 2048, 0, WIDE, WIDE),
     # 33 to 64 rows: 32 rows by 32 columns; past K = 4096 only where its workgroups do not split K, past
     # 4608 only where the row groups share an XCD (a multiple of eight column groups)
-    (33, 4096, 4096, 0, GENERIC), (33, 4097, 4096, 0, WIDE), (64, 2048, 4608, 0, GENERIC), (64, 2016, 4608, 0, WIDE),
-    (64, 2080, 4608, 0, GENERIC), (64, 2080, 4736, 0, WIDE), (64, 2304, 7424, 0, GENERIC), (64, 2304, 7552, 0, WIDE),
+    (33, 4096, 4096, 0, GENERIC, GENERIC), (33, 4097, 4096, 0, WIDE, WIDE), (64, 2048, 4608, 0, GENERIC, GENERIC),
+    (64, 2016, 4608, 0, WIDE, WIDE), (64, 2080, 4608, 0, GENERIC, GENERIC), (64, 2080, 4736, 0, WIDE, WIDE),
+    (64, 2304, 6144, 0, GENERIC, GENERIC), (64, 2304, 6272, 0, WIDE, GENERIC), (64, 2304, 7424, 0, WIDE, GENERIC),
+    (64, 2304, 7552, 0, WIDE, WIDE),
     # more: 64 rows by 16 columns
-    (65, 2048, 4096, 0, GENERIC), (65, 2049, 4096, 0, WIDE), (65, 2048, 4352, 0, GENERIC), (65, 2032, 4352, 0, WIDE),
-    (65, 2048, 5376, 0, GENERIC), (65, 2048, 5504, 0, WIDE), (65, 1536, 5376, 0, GENERIC), (65, 1408, 4480, 0, WIDE),
-    (640, 400, 2176, 0, GENERIC), (641, 256, 3200, 0, WIDE), (1280, 192, 3072, 0, GENERIC),
-    (1281, 128, 2176, 0, WIDE),
+    (65, 2048, 4096, 0, GENERIC, GENERIC), (65, 2049, 4096, 0, WIDE, WIDE), (65, 2048, 4352, 0, GENERIC, GENERIC),
+    (65, 2032, 4352, 0, WIDE, WIDE), (65, 2048, 5376, 0, GENERIC, GENERIC), (65, 2048, 5504, 0, WIDE, WIDE),
+    (65, 1536, 5376, 0, GENERIC, GENERIC), (65, 1408, 4480, 0, WIDE, WIDE), (512, 512, 5376, 0, GENERIC, GENERIC),
+    (513, 384, 5376, 0, WIDE, WIDE), (513, 384, 4352, 0, GENERIC, GENERIC), (640, 400, 2176, 0, GENERIC, GENERIC),
+    (641, 256, 3200, 0, WIDE, WIDE), (1024, 192, 3072, 0, GENERIC, GENERIC), (1025, 192, 2688, 0, WIDE, WIDE),
+    (1280, 192, 2560, 0, GENERIC, GENERIC), (1281, 128, 2176, 0, WIDE, WIDE),
     # block-FP8
-    (32, 4096, 4608, 1, GENERIC), (32, 4096, 4736, 1, WIDE), (64, 4096, 4352, 1, GENERIC), (64, 4064, 4352, 1, WIDE),
-    (64, 4064, 2176, 1, GENERIC), (65, 128, 2176, 1, WIDE), (17, 8192, 2048, 1, WIDE),
+    (32, 4096, 4608, 1, GENERIC, None), (32, 4096, 4736, 1, WIDE, None), (64, 4096, 4352, 1, GENERIC, None),
+    (64, 4064, 4352, 1, WIDE, None), (64, 4064, 2176, 1, GENERIC, None), (65, 128, 2176, 1, WIDE, None),
+    (17, 8192, 2048, 1, WIDE, None),
 ])
-def test_one_round_of_the_generic_kernel(pkg, M, N, K, block, kernel):
-    assert _plan(M, N, K, 0, block).startswith(kernel)
-    if kernel == GENERIC:
+def test_one_round_of_the_generic_kernel(pkg, M, N, K, block, mxfp8, mxfp6):
+    assert _plan(M, N, K, 0, block).startswith(mxfp8)
+    if mxfp8 == GENERIC:
         assert not _plan(M, N, K, 0, block).endswith("reduce8_kernel") or K > 4096
     if not block:
-        assert _plan(M, N, K, 2).startswith(kernel) and _plan(M, N, K, 3).startswith(kernel)
+        assert _plan(M, N, K, 2).startswith(mxfp6) and _plan(M, N, K, 3).startswith(mxfp6)
 
 
 def test_kept_plans_are_the_plans_of_their_sizes(pkg):

@@ -565,29 +565,34 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
 // than the CUs there, walk K alone or split it through partials and a second launch.  Measured over
 // 9000 shapes of 17 to 4096 rows (generic against tiles, share of the tiles' time; one more round
 // costs the generic kernel 20 to 60 %):
-//   up to 32 rows, MX: K = 896 0.88 to 0.92 (up to 768 0.94 to 1.07), 2176 to 8192 0.65 to 1.05 (18 x 2672
-//     x 3072 5.8 us against 8.8, 24 x 2560 x 6272 7.9 against 12.0), up to 9088 unsplit or of at most 64
-//     workgroups 0.88 to 0.99 (otherwise up to 1.22); block-FP8 2176 to 4608 0.72 to 0.95 (24 x 3072 x 3072 7.2 against 9.3; from 4736 0.94 to 1.10)
+//   up to 32 rows, MX: K = 896 0.87 to 0.96 (up to 768 0.94 to 1.07), 2176 to 8192 0.63 to 1.05 (18 x 2672
+//     x 3072 5.8 us against 8.8, 24 x 2560 x 6272 7.9 against 12.0), MXFP6 up to 9088 unsplit or of at most
+//     64 workgroups 0.91 to 1.09, mean 0.98 (MXFP8 0.96 to 1.15, mean 1.06); block-FP8 2176 to 4608 0.72 to
+//     0.95 (24 x 3072 x 3072 7.2 against 9.3; from 4736 0.94 to 1.10)
 //   33 to 64 rows (two row groups, which share their weights in an XCD's L2 where the column groups
 //     are a multiple of eight), MX: 2176 to 4096 0.75 to 1.02 (43 x 3840 x 2560 7.1 against 8.5), up to 4608
-//     unsplit 0.84 to 0.95, up to 7424 shared 0.80 to 0.99 (otherwise 0.90 to 1.26); block-FP8 up to 4096
-//     0.79 to 1.05, up to 4352 shared 0.85 to 0.89 (past it 0.98 to 1.44)
-//   65 to 640 rows, MX: 2176 to 4096 0.80 to 1.06 (200 x 1024 x 3328 8.1 against 9.2), up to 4352 unsplit
-//     shared 0.89 to 0.99 (past it 0.91 to 1.67), up to 5376 shared by at least 3/4 of the CUs 0.91 to 1.04
-//     (256 x 1024 x 4480 9.8 against 10.6, 180 x 1280 x 5248 11.3 both, and one launch for two); up to 1280 rows
-//     2176 to 3072 0.80 to 1.03 (past it up to 1.37).  Block-FP8 from 65 rows 1.03 to 1.17 and more.
+//     unsplit 0.84 to 0.95, shared up to 6144 (MXFP8) 0.85 to 1.03 and 7424 (MXFP6) 0.74 to 1.05 (past them
+//     1.02 to 1.11, unshared 0.90 to 1.26); block-FP8 up to 4096 0.79 to 1.05, up to 4352 shared 0.85 to 0.89
+//     (past it 0.98 to 1.44)
+//   65 to 640 rows, MX: 2176 to 4096 0.74 to 1.06 (200 x 1024 x 3328 8.1 against 9.2), up to 4352 unsplit
+//     shared 0.88 to 1.04 (past it 0.91 to 1.67), up to 512 rows to 5376 shared by at least 3/4 of the CUs
+//     0.91 to 1.08, mean 0.98 (256 x 1024 x 4480 9.8 against 10.6, 180 x 1280 x 5248 11.3 both, and one launch
+//     for two; 640 x 384 x 5376 1.28); up to 1024 rows 2176 to 3072 0.78 to 1.03, up to 1280 to 2560
+//     0.80 to 0.98 (at 3072 1.03 to 1.08).  Block-FP8 from 65 rows 1.03 to 1.17 and more.
 // Two workgroups per CU are one round too at 17 to 32 rows and K = 1024 to 2048, MX: 0.87 to 0.97
 // (31 x 6656 x 1920 6.5 us against 7.5; with more of them 1.07 to 1.58).
-static bool generic_round(int64_t M, int64_t N, int64_t K, bool block) {
+static bool generic_round(int64_t M, int64_t N, int64_t K, int fmt, bool block) {
   const GemmConfig c = choose_config(M, N, K);
   const int64_t n_groups = ((N + 15) / 16 + c.NT - 1) / c.NT, m_groups = (M + 16 * c.MT - 1) / (16 * c.MT);
   const int64_t groups = n_groups * m_groups, cus = cu_count();
-  const bool unsplit = c.S == 1, shared = unsplit && n_groups % 8 == 0;
+  const bool unsplit = c.S == 1, shared = unsplit && n_groups % 8 == 0, fp6 = fmt != kE4M3;
   if (!block && M <= 32 && K >= 1024 && K <= 2048) return groups <= 2 * cus;
   if (groups > cus || K <= (!block && M <= 32 ? 768 : 2048)) return false;
-  if (M <= 32) return K <= (block ? 4608 : unsplit || groups <= 64 ? 9088 : 8192);
-  if (M <= 64) return K <= (block ? (shared ? 4352 : 4096) : shared ? 7424 : unsplit ? 4608 : 4096);
-  return !block && (M <= 640 ? K <= (!shared ? 4096 : 4 * groups >= 3 * cus ? 5376 : 4352) : M <= 1280 && K <= 3072);
+  if (M <= 32) return K <= (block ? 4608 : fp6 && (unsplit || groups <= 64) ? 9088 : 8192);
+  if (block) return M <= 64 && K <= (shared ? 4352 : 4096);
+  if (M <= 64) return K <= (shared ? (fp6 ? 7424 : 6144) : unsplit ? 4608 : 4096);
+  if (M <= 640) return K <= (!shared ? 4096 : M <= 512 && 4 * groups >= 3 * cus ? 5376 : 4352);
+  return K <= (M <= 1024 ? 3072 : M <= 1280 ? 2560 : 0);
 }
 
 // An automatic plan is a function of the sizes, the weight and the CUs, and a call asks for it up to four
@@ -645,7 +650,7 @@ static bool plan_dense_as(int64_t M, int64_t N, int64_t K, int fmt, bool block, 
   const bool generic_pref =
       (!block && M > 32 && M <= (tiles_ok ? 128 : 256) && K >= 1024 && K <= 2048 && (N + 15) / 16 <= 128) ||
       (M < 64 && K >= 1024 && N * K <= (K <= 2048 ? int64_t(12) << 20 : K <= 4096 ? int64_t(4) << 20 : 0)) ||
-      (tiles_ok && generic_round(M, N, K, block));
+      (tiles_ok && generic_round(M, N, K, fmt, block));
   d.kernel = o.kernel == kAuto
                  ? (stream_ok                                        ? kStream
                     : chunk_pref                                     ? kChunk
