@@ -100,7 +100,8 @@ def test_kept_plans_are_the_plans_of_their_sizes(pkg):
 
 
 @pytest.mark.parametrize("M,N,K,block", [(749, 6400, 1024, 0), (1002, 4688, 1024, 0), (637, 8152, 1536, 0),
-                                         (256, 18432, 1024, 0), (793, 5504, 2432, 1), (2048, 2560, 9216, 0)])
+                                         (256, 18432, 1024, 0), (793, 5504, 2432, 1), (197, 17920, 3584, 1),
+                                         (2048, 2560, 9216, 0)])
 def test_a_part_round_of_tiles_runs_in_one_launch(pkg, M, N, K, block):
     """Up to 64 tiles of 128 x 128 past one round of the CUs: their quarters beside the whole tiles, not a K
     split and its reduce (2 to 5 us slower at each of these)."""

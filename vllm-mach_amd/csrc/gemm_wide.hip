@@ -1,6 +1,8 @@
 // Wide-tile, LDS-pipelined GEMM for prefill-sized M on gfx950 (MX and block-FP8,
 // dense): the four-wave tiles, the planner of the dense 2 x 2-wave tiles
 // (gemm_tile.hip; what the automatic dense plans run) and the split reduce of both.
+// The four-wave tiles run where a call's options or a registered entry set a tile, split or
+// wave field (waves = 8 aside), and are the bit reference that the tests hold the others to.
 //
 // Workgroup tile: 128 rows x 64*NT columns (NT = 1, 2 or 4), four wavefronts.
 // Every wave owns all 8 m-tiles of the 128 rows and its own NT n-tiles; per
@@ -763,9 +765,8 @@ WideConfig wide_config(int64_t M, int64_t N, int64_t K, int fmt, const GemmOptio
 // MXFP8, MXFP6 and block-FP8 weights rotated out of the caches: a launch costs its fixed time, the
 // stages of the fullest CU, and its output, which nothing overlaps in the last round.  What all
 // choices share is left out (the operands' way from memory), so it is some 7 % low on average.  The
-// plans of 1103 shapes run within 1.0 % of the best tile and split on average (the farthest of its
-// picks: 200 x 16640 x 512 12.0 us against 9.0, 3912 x 2208 x 512 15.5 against 12.1, 1470 x 2816 x 5760
-// 40.4 against 34.0).
+// plans of 700 drawn shapes run within 1.6 % of the best tile and split on average (the farthest of its
+// picks: 548 x 7608 x 768 12.0 us against 9.6, 3119 x 1528 x 512 10.0 against 8.0).
 struct TileCost {
   int MT, NT, resident;   // tile, workgroups per CU
   double fixed, stage;    // us: of the launch, of a K128 stage on one CU
@@ -800,11 +801,15 @@ static int64_t wide_tail(const TileCost& t, int64_t tiles, int64_t cus) {
 }
 
 // Up to two blocks of 128 rows the weights' way from memory sets the pace, and over a long K the
-// hybrid's units end beside the whole tiles: MX from K = 5120 it runs even with the quarters or ahead
-// (160 / 256 x 16640 / 17408 x 5120 36.0 / 40.4 us against 39.7 / 40.3, 200 x 16640 x 8192 47.7 against
-// 53.7; 256 x 18432 x 4096 35.6 against 32.4).  Block-FP8 gives up 2 to 14 % there to keep the plan of
-// its gate_up layer, which is held by name (256 x 18432 x 2560 27.8 against 23.9).
-static bool hybrid_kept(int64_t M, int64_t K, bool block) { return M <= 256 && K >= (block ? 2560 : 5120); }
+// hybrid's units end beside the whole tiles: from K = 5120 it runs even with the quarters or ahead (MX
+// 160 / 256 x 16640 / 17408 x 5120 36.0 / 40.4 us against 39.7 / 40.3, 200 x 16640 x 8192 47.7 against 53.7;
+// block-FP8 256 x 16640 x 5120 38.8 against 39.9, 256 x 18432 x 8192 60.8 against 59.8), below it behind
+// (256 x 18432 x 4096 35.6 against 32.4; block-FP8 197 x 17920 x 3584 34.3 against 27.7).  Block-FP8 keeps it
+// at K = 2560 to 2944 for the plan of its gate_up layer, which is held by name (256 x 18432 x 2560 27.8
+// against 23.9).
+static bool hybrid_kept(int64_t M, int64_t K, bool block) {
+  return M <= 256 && (K >= 5120 || (block && K >= 2560 && K < 3072));
+}
 
 bool wide_tiles_eligible(int64_t M, int64_t N, int64_t K, bool block) {
   // 32-bit operand offsets
