@@ -164,9 +164,9 @@ typedef struct mxl_gemm_options {
   int hybrid;    /* wide, splits == 1: whole-K full rounds, the remainder split */
   int waves;     /* wide dense with 128-row tiles: 4 waves per CU (one workgroup, each wave
                     all 128 rows) or 8 (two workgroups of 2 x 2 waves, each wave half the
-                    rows and columns); 0 automatic.  With kernel -1 and the five tile
-                    and split fields automatic a call of more than 16 rows also has the 64-
-                    and 256-row 2 x 2-wave tiles to choose from, at any K % 128 == 0 */
+                    rows and columns); 0 automatic.  With the five tile and split fields
+                    automatic a wide call takes 2 x 2-wave tiles of 64 to 256 rows; with
+                    kernel -1 as well from 17 rows on and at any K % 128 == 0 */
   int out_dtype; /* output elements: 0 bf16, 1 fp16 (dense GEMMs; the grouped and
                     two-limb GEMMs write bf16 only) */
   float alpha;   /* output scale: out = round(alpha * sum) with the fp32 sum scaled

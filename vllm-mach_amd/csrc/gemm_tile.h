@@ -1,5 +1,5 @@
 // One output tile of the 2 x 2-wave GEMM on gfx950 (MX and block-FP8 weights): the device
-// body of gemm_tile.hip's kernels and of the wide kernel's 128 x 128 tiles (gemm_wide.hip).
+// body of the dense kernels of gemm_tile.hip and the grouped ones of gemm_tile_grouped.hip.
 //
 // What bounds it.  At 128 x 128 tiles per workgroup every K128 stage moves as many LDS
 // bytes as the LDS serves in the time of its MFMAs, so the wide kernel (gemm_wide.hip)
@@ -25,8 +25,10 @@
 // they do not run, the generic kernel before): W6A8 4096 x 17408 x 5120 665 -> 302 (2.4 PFLOP/s),
 // 1024 x 17408 x 5120 150 -> 95, 48 x 17408 x 5120 51 -> 23.4 (2.9 TB/s of weights); block-FP8 512
 // x 18432 x 2560 55.5 -> 36.2, 32 x 18432 x 2560 29.3 -> 13.5 (3.5 TB/s); MXFP8 512 x 2560 x 9216
-// 27.9 -> 25.8.  The 256 x 256 tile is bound by its MFMAs (without copies or LDS reads its stages
-// took 13 % less); the smaller ones by their LDS traffic and, in the last round, the epilogue.
+// 27.9 -> 25.8.  The 256 x 256 tile is bound by its MFMAs at the clock that the power limit leaves (W6A8
+// 4096 x 17408 x 5120: MFMAs busy 58 % of the cycles, 0.6 LDS reads each), the smaller ones by their LDS
+// traffic (1.3 to 1.7 reads per MFMA; 8-byte FP6 reads with bank conflicts) and, in the last round, the
+// epilogue.
 //
 // The weights take the MFMA's A operand and the activations its B operand, so a lane holds
 // four consecutive output columns of one row (8-byte stores), and in block-FP8 its four
